@@ -345,33 +345,41 @@ struct Mrt3 {
   
 };
 
-template <int K>
-__device__ __forceinline__ float int_row(const int (&row)[K], const float (&x)[K]) {
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < K; ++i) {
-    const int m = row[i];
-    if (m == 1) s += x[i];
-    else if (m == -1) s -= x[i];
-    else if (m != 0) s += (float)m * x[i];
+// sum_i T[k][i] x[i] of an integer table T: the entries are read as constants
+// at each use, so that an unrolled call folds into adds and multiply-adds.
+// (Passed as a row reference, the table stayed in memory: each entry was then
+// loaded and branched on at run time, some 5000 branches per cell: 20 steps of
+// a 121 x 113 x 127 MRT cavity took 27.1 ms that way, 3.19 ms since.)
+#define VSX_INT_ROW(name, T)                                       \
+  __device__ __forceinline__ float name(int k, const float (&x)[19]) { \
+    float s = 0.f;                                                 \
+    _Pragma("unroll") for (int i = 0; i < 19; ++i) {               \
+      const int m = T[k][i];                                       \
+      if (m == 1) s += x[i];                                       \
+      else if (m == -1) s -= x[i];                                 \
+      else if (m != 0) s += (float)m * x[i];                       \
+    }                                                              \
+    return s;                                                      \
   }
-  return s;
-}
+VSX_INT_ROW(mrow3, Mrt3::M)
+VSX_INT_ROW(nrow3, Mrt3::N72)
+#undef VSX_INT_ROW
 
-// f += M^-1 [ S M (feq - f) + (I - S/2) M F ]  (F == nullptr -> collision only)
-__device__ __forceinline__ void mrt_d3q19(float (&f)[19], const float (&feq)[19], const float (&F)[19], bool has_f,
+// f += M^-1 [ S M (feq - f) + (I - S/2) M F ]  (HAS_F false -> collision only)
+template <bool HAS_F>
+__device__ __forceinline__ void mrt_d3q19(float (&f)[19], const float (&feq)[19], const float (&F)[19],
                                           const float *rates) {
   float d[19], r[19];
 #pragma unroll
   for (int i = 0; i < 19; ++i) d[i] = feq[i] - f[i];
 #pragma unroll
   for (int k = 0; k < 19; ++k) {
-    float v = rates[k] * int_row<19>(Mrt3::M[k], d);
-    if (has_f) v += (1.f - 0.5f * rates[k]) * int_row<19>(Mrt3::M[k], F);
+    float v = rates[k] * mrow3(k, d);
+    if (HAS_F) v += (1.f - 0.5f * rates[k]) * mrow3(k, F);
     r[k] = v;
   }
 #pragma unroll
-  for (int i = 0; i < 19; ++i) f[i] += int_row<19>(Mrt3::N72[i], r) * (1.f / 72.f);
+  for (int i = 0; i < 19; ++i) f[i] += nrow3(i, r) * (1.f / 72.f);
 }
 
 }  // namespace vsx

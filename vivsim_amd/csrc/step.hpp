@@ -336,7 +336,8 @@ __device__ __forceinline__ void collide_force(float (&f)[L::Q], float rho, const
       }
     } else {
       forced = has_g && forcing == VSX_FORCE_GUO;
-      mrt_d3q19(f, feq, F, forced, rates);
+      if (forced) mrt_d3q19<true>(f, feq, F, rates);
+      else mrt_d3q19<false>(f, feq, F, rates);
     }
   }
   if (has_g && !forced) {
