@@ -19,9 +19,8 @@
 // neighbour line) and the last writer wins at corners.  A cell on exactly one
 // wall whose update reads no cell rewritten by an earlier wall is finished in
 // the bulk kernel (one extra pull for the neighbour line).  The remaining cells
-// (corners and corner-adjacent cells of perpendicular wall pairs) go to a
-// separate edge kernel that replays the wall list recursively (depth <= number
-// of walls); it is launched only when such cells can exist.
+// (on walls of several axes) go to the first blocks of the same launch, a group
+// of 2^D lanes per cell (edge_cells); they exist only when such cells do.
 #pragma once
 #include <type_traits>
 #include <utility>
@@ -118,15 +117,6 @@ __device__ __forceinline__ int64_t wall_node(const StepCtx &c, int loc, const in
   return (int64_t)co[0] * c.dims[1] + co[1];
 }
 
-template <class L>
-__device__ __forceinline__ bool on_any_wall(const StepCtx &c, const int (&co)[3], int upto) {
-  bool on = false;
-#pragma unroll
-  for (int k = 0; k < L::n_walls; ++k)
-    if (k < upto) on |= on_wall<L>(c, c.p.walls[k].loc, co);
-  return on;
-}
-
 // Post-streaming, post-walls populations of cell co after walls [0, J).
 // TAG only separates instantiations: an out-of-line function takes its register
 // budget from the kernels that call it, so a kernel with a tight budget calls
@@ -175,8 +165,7 @@ __device__ __forceinline__ bool on_wall_at(const StepCtx &c, const int (&co)[3])
 // Wall class of a cell: -1 on no wall; LOC when the cell is on exactly one wall
 // (at location LOC) and that wall reads no neighbour rewritten by an earlier
 // wall, so one pull and one wall update reproduce the ordered sequence; -2
-// otherwise (corners and corner-adjacent cells, replayed recursively by the
-// edge kernel).
+// otherwise (cells on walls of several axes, left to edge_cells).
 template <class L>
 __device__ __forceinline__ int wall_class(const StepCtx &c, const int (&co)[3]) {
   int loc_on = -1, count = 0;
@@ -387,23 +376,116 @@ __device__ __forceinline__ void finish(const StepCtx &c, uint32_t cell, const in
   collide_force<L, COLL>(f, rho, u, g, c.p.forcing, c.p.omega, c.p.mrt_rates);
 }
 
+// ------------------------------------------------------------------ cells on several walls
+// Lines of cells on the walls of two axes, and whole faces that carry two
+// walls (host list, make_edges).
+constexpr int kMaxEdges = 16;
+struct EdgeList {
+  int32_t n = 0;                   // entries
+  int32_t loc[kMaxEdges][2];       // an edge: the two faces; a face: {loc, -1}
+  int64_t begin[kMaxEdges + 1];    // first cell of each entry
+};
+
+// The cells of wall class -2.  The state of such a cell after wall w needs the
+// state of its inward neighbour across w after the walls before w, and so on:
+// for a cell on the walls of m axes, the 2^m cells reached by moving inward
+// along any of these axes.  A group of 2^D lanes holds them, lane bit a set =
+// moved inward along axis a; every lane pulls its own cell, then the walls are
+// taken in list order, each lane on the wall reading its neighbour's populations
+// from the lane of that bit.  Replayed by one thread as a recursion over the walls
+// (scratch arrays, one chain of loads per level) these cells took 17 us of a
+// 256^2 cavity step and 120 us of a 121 x 113 x 127 one, as a kernel of their own.
+template <class L, int COLL, int PHASE, class SRC, class DST>
+__device__ __forceinline__ void edge_cells(const StepCtx &c, const EdgeList &E, int64_t t,
+                                           const typename SRC::T *__restrict__ src,
+                                           typename DST::T *__restrict__ dst) {
+  constexpr int G = 1 << L::D;
+  const int member = (int)(t % G);
+  int64_t j = t / G;
+  bool active = j < E.begin[E.n];
+  int e = 0;
+  for (int k = 1; k < E.n; ++k) e = j >= E.begin[k] ? k : e;
+  j = active ? j - E.begin[e] : 0;
+  int co[3] = {0, 0, 0};
+  const int la = E.loc[e][0], lb = E.loc[e][1];
+  const int a = L::w_axis[la], b = lb >= 0 ? L::w_axis[lb] : -1;
+  // the free axes, fastest last (2D: axis 2 has one cell)
+#pragma unroll
+  for (int ax = 2; ax >= 0; --ax) {
+    if (ax == a) {
+      co[ax] = L::w_sign[la] > 0 ? 0 : c.dims[ax] - 1;
+    } else if (ax == b) {
+      co[ax] = L::w_sign[lb] > 0 ? 0 : c.dims[ax] - 1;
+    } else {
+      co[ax] = (int)(j % c.dims[ax]);
+      j /= c.dims[ax];
+    }
+  }
+  // inward direction per axis (0: on no wall of that axis)
+  int s[3] = {0, 0, 0}, cn[3];
+  static_for<L::n_walls>([&](auto LC) {
+    constexpr int LOC = decltype(LC)::value;
+    if (c.order[LOC] != -1 && on_wall_at<L, LOC>(c, co)) s[L::w_axis[LOC]] = L::w_sign[LOC];
+  });
+  // a cell on the walls of three axes is taken with the edge of axes 0 and 1,
+  // a face's border with the edges
+  if (b < 0) active = active && (s[0] != 0) + (s[1] != 0) + (s[2] != 0) == 1;
+  else if (a + b != 1) active = active && !(s[0] && s[1] && s[2]);
+#pragma unroll
+  for (int ax = 0; ax < 3; ++ax) cn[ax] = co[ax] + ((member >> ax) & 1 ? s[ax] : 0);
+  const uint32_t cell = cell_of<L>(c, cn[0], cn[1], cn[2]);
+  float f[L::Q];
+  pull<L, SRC>(c, src, cn[0], cn[1], cn[2], f);
+  for (int k = 0; k < c.p.n_walls; ++k) {
+    const VsxWall &w = c.p.walls[k];
+    const int ax = L::w_axis[w.loc], sg = L::w_sign[w.loc];
+    const bool on = comp3(s, ax) == sg && !((member >> ax) & 1);
+    float fn[L::Q], fp[L::Q];
+#pragma unroll
+    for (int i = 0; i < L::Q; ++i) fn[i] = fp[i] = 0.f;
+    if (wall_needs_neighbor(w)) {
+#pragma unroll
+      for (int i = 0; i < L::Q; ++i) fn[i] = __shfl_xor(f[i], 1 << ax, 64);
+    }
+    if (on) {
+      if (wall_needs_pre(w)) local<L, SRC>(c, src, cell, fp);
+      apply_wall<L>(w, wall_node<L>(c, w.loc, cn), f, fn, fp);
+    }
+  }
+  if (!active || member != 0) return;
+  if constexpr (PHASE == VSX_PHASE_FULL) {
+    int org[3];
+    const bool win = window_origin_of<L>(c, org);
+    finish<L, COLL>(c, cell, cn, org, win, f);
+  }
+  store_cell<L, DST>(c, dst, cell, f);
+}
+
 // ------------------------------------------------------------------ kernels
 // Bulk: one thread per cell; blockIdx.x tiles the contiguous axis, blockIdx.y
 // (and z in 3D) the others, so a wavefront touches 64 consecutive cells.
+// EDGE: the first `edge_rows` rows of the outermost grid axis hold the cells on
+// several walls.  Their long chains (a few waves) run beside the bulk, and the
+// kernel keeps the register budget of the bulk path (waves_per_eu): what the
+// edge path needs above it is spilled there.
+template <class L>
+constexpr int bulk_waves() {
+  return L::D == 2 ? 8 : 5;
+}
+
 template <class L, int COLL, int PHASE, class SRC, class DST>
-__global__ __launch_bounds__(256) void k_bulk(StepCtx c_arg, const typename SRC::T *__restrict__ src,
-                                              typename DST::T *__restrict__ dst) {
-  const StepCtx &c = kernel_ctx();
+__device__ __forceinline__ void bulk_cells(const StepCtx &c, int outer, const typename SRC::T *__restrict__ src,
+                                           typename DST::T *__restrict__ dst) {
   int co[3];
   if constexpr (L::D == 2) {
     co[1] = blockIdx.x * blockDim.x + threadIdx.x;
-    co[0] = blockIdx.y;
+    co[0] = outer;
     co[2] = 0;
     if (co[1] >= c.dims[1]) return;
   } else {
     co[2] = blockIdx.x * blockDim.x + threadIdx.x;
     co[1] = blockIdx.y;
-    co[0] = blockIdx.z;
+    co[0] = outer;
     if (co[2] >= c.dims[2]) return;
   }
   const uint32_t cell = cell_of<L>(c, co[0], co[1], co[2]);
@@ -417,7 +499,7 @@ __global__ __launch_bounds__(256) void k_bulk(StepCtx c_arg, const typename SRC:
     if (cls != -1) {
       // wall cell: a separate path (own finish and store) keeps the wall code's
       // register demand out of the interior path below
-      if (cls < 0) return;   // corner cells: edge kernel
+      if (cls < 0) return;   // cells on several walls: edge_cells
       single_wall_state<L, SRC>(c, src, co, cls, f);
       if constexpr (PHASE != VSX_PHASE_STREAM) finish<L, COLL>(c, cell, co, org, win, f);
       store_cell<L, DST>(c, dst, cell, f);
@@ -429,48 +511,25 @@ __global__ __launch_bounds__(256) void k_bulk(StepCtx c_arg, const typename SRC:
   store_cell<L, DST>(c, dst, cell, f);
 }
 
-// Edge: the cells of wall class -2, enumerated as (wall, node) pairs; a cell on
-// several walls is handled under the first wall (in list order) that contains it.
-template <class L, int PHASE, class SRC, class DST>
-__global__ __launch_bounds__(256) void k_edge(StepCtx c_arg, const typename SRC::T *__restrict__ src,
-                                              typename DST::T *__restrict__ dst, int64_t per_wall) {
+template <class L, int COLL, int PHASE, class SRC, class DST>
+__global__ __launch_bounds__(256) void k_bulk(StepCtx c_arg, const typename SRC::T *__restrict__ src,
+                                              typename DST::T *__restrict__ dst) {
+  bulk_cells<L, COLL, PHASE, SRC, DST>(kernel_ctx(), L::D == 2 ? blockIdx.y : blockIdx.z, src, dst);
+}
+
+template <class L, int COLL, int PHASE, class SRC, class DST>
+__global__ __attribute__((amdgpu_flat_work_group_size(64, 256),
+                          amdgpu_waves_per_eu(bulk_waves<L>(), bulk_waves<L>()))) void
+k_bulk_edge(StepCtx c_arg, const typename SRC::T *__restrict__ src, typename DST::T *__restrict__ dst, EdgeList E,
+            int edge_rows) {
   const StepCtx &c = kernel_ctx();
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int k = (int)(t / per_wall);
-  const int64_t j = t % per_wall;
-  if (k >= c.p.n_walls) return;
-  const int loc = c.p.walls[k].loc, a = L::w_axis[loc];
-  int co[3];
-  // node j -> coordinates on the wall (same order as the per-node arrays)
-  int b0 = a == 0 ? 1 : 0, b1 = a == 2 ? 1 : 2;
-  const int n1 = L::D == 2 ? 1 : c.dims[b1];
-  const int64_t nodes = (int64_t)c.dims[b0] * (L::D == 2 ? 1 : c.dims[b1]);
-  if (L::D == 2) { b0 = 1 - a; b1 = 2; }
-  if (j >= (L::D == 2 ? (int64_t)c.dims[1 - a] : nodes)) return;
-  co[a] = L::w_sign[loc] > 0 ? 0 : c.dims[a] - 1;
-  if constexpr (L::D == 2) {
-    co[1 - a] = (int)j;
-    co[2] = 0;
-  } else {
-    co[b0] = (int)(j / n1);
-    co[b1] = (int)(j % n1);
+  const int outer = L::D == 2 ? blockIdx.y : blockIdx.z;
+  if (outer < edge_rows) {
+    const int64_t row = L::D == 2 ? (int64_t)outer : (int64_t)outer * gridDim.y + blockIdx.y;
+    edge_cells<L, COLL, PHASE, SRC, DST>(c, E, (row * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x, src, dst);
+    return;
   }
-  if (on_any_wall<L>(c, co, k)) return;     // handled under the first wall that contains it
-  if (wall_class<L>(c, co) != -2) return;   // bulk kernel
-  const uint32_t cell = cell_of<L>(c, co[0], co[1], co[2]);
-  float f[L::Q];
-  wall_state<L, SRC, L::n_walls>(c, src, co, f);
-  if constexpr (PHASE == VSX_PHASE_FULL) {
-    int org[3];
-    const bool win = window_origin_of<L>(c, org);
-    switch (c.p.collision) {
-      case VSX_COLL_BGK: finish<L, VSX_COLL_BGK>(c, cell, co, org, win, f); break;
-      case VSX_COLL_MRT: finish<L, VSX_COLL_MRT>(c, cell, co, org, win, f); break;
-      case VSX_COLL_KBC: finish<L, VSX_COLL_KBC>(c, cell, co, org, win, f); break;
-      default: finish<L, VSX_COLL_REG>(c, cell, co, org, win, f); break;
-    }
-  }
-  store_cell<L, DST>(c, dst, cell, f);
+  bulk_cells<L, COLL, PHASE, SRC, DST>(c, outer - edge_rows, src, dst);
 }
 
 }  // namespace vsx

@@ -63,17 +63,47 @@ void bulk_grid(const StepCtx &c, dim3 &grid, dim3 &block) {
   else grid = dim3((inner + b - 1) / b, c.dims[1], c.dims[0]);
 }
 
+// The lines and faces of edge_cells: every pair of walled faces of two axes, and
+// every face with two walls.
 template <class L>
-int64_t edge_per_wall(const StepCtx &c) {
-  int64_t m = 0;
-  for (int k = 0; k < c.p.n_walls; ++k) {
-    const int a = L::w_axis[c.p.walls[k].loc];
-    int64_t nodes = 1;
-    for (int b = 0; b < L::D; ++b)
-      if (b != a) nodes *= c.dims[b];
-    if (nodes > m) m = nodes;
+EdgeList make_edges(const StepCtx &c) {
+  EdgeList E;
+  int64_t cells = 0;
+  auto add = [&](int la, int lb) {
+    const int a = L::w_axis[la], b = lb >= 0 ? L::w_axis[lb] : -1;
+    int64_t m = 1;
+    for (int k = 0; k < 3; ++k)
+      if (k != a && k != b) m *= c.dims[k];
+    E.loc[E.n][0] = la;
+    E.loc[E.n][1] = lb;
+    E.begin[E.n++] = cells;
+    cells += m;
+  };
+  for (int la = 0; la < L::n_walls; ++la) {
+    if (c.order[la] == -1) continue;
+    for (int lb = la + 1; lb < L::n_walls; ++lb)
+      if (c.order[lb] != -1 && L::w_axis[lb] != L::w_axis[la]) add(la, lb);
+    if (c.order[la] == -2) add(la, -1);
   }
-  return m;
+  E.begin[E.n] = cells;
+  return E;
+}
+
+template <class L, int COLL, int PHASE, class SRC, class DST>
+void launch_bulk(const StepCtx &c, const typename SRC::T *src, typename DST::T *dst, dim3 grid, dim3 block,
+                 hipStream_t s) {
+  if constexpr (PHASE != VSX_PHASE_COLLIDE) {
+    if (c.p.n_walls > 0 && walls_need_edge<L>(c.p)) {
+      const EdgeList E = make_edges<L>(c);
+      const int64_t blocks = ((E.begin[E.n] << L::D) + block.x - 1) / block.x;
+      const int64_t per_row = (int64_t)grid.x * (L::D == 2 ? 1 : grid.y);
+      const int rows = (int)((blocks + per_row - 1) / per_row);
+      (L::D == 2 ? grid.y : grid.z) += rows;
+      hipLaunchKernelGGL((k_bulk_edge<L, COLL, PHASE, SRC, DST>), grid, block, 0, s, c, src, dst, E, rows);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_bulk<L, COLL, PHASE, SRC, DST>), grid, block, 0, s, c, src, dst);
 }
 
 template <class L, int PHASE, class SRC, class DST>
@@ -84,23 +114,16 @@ int launch_phase(const StepCtx &c, const void *src, void *dst, hipStream_t s) {
   auto D = static_cast<typename DST::T *>(dst);
   if constexpr (PHASE == VSX_PHASE_FULL) timer_begin(s);
   if constexpr (PHASE == VSX_PHASE_STREAM) {
-    hipLaunchKernelGGL((k_bulk<L, VSX_COLL_BGK, PHASE, SRC, DST>), grid, block, 0, s, c, S, D);
+    launch_bulk<L, VSX_COLL_BGK, PHASE, SRC, DST>(c, S, D, grid, block, s);
   } else {
     switch (c.p.collision) {
-      case VSX_COLL_BGK: hipLaunchKernelGGL((k_bulk<L, VSX_COLL_BGK, PHASE, SRC, DST>), grid, block, 0, s, c, S, D); break;
-      case VSX_COLL_MRT: hipLaunchKernelGGL((k_bulk<L, VSX_COLL_MRT, PHASE, SRC, DST>), grid, block, 0, s, c, S, D); break;
-      case VSX_COLL_KBC: hipLaunchKernelGGL((k_bulk<L, VSX_COLL_KBC, PHASE, SRC, DST>), grid, block, 0, s, c, S, D); break;
-      default: hipLaunchKernelGGL((k_bulk<L, VSX_COLL_REG, PHASE, SRC, DST>), grid, block, 0, s, c, S, D); break;
+      case VSX_COLL_BGK: launch_bulk<L, VSX_COLL_BGK, PHASE, SRC, DST>(c, S, D, grid, block, s); break;
+      case VSX_COLL_MRT: launch_bulk<L, VSX_COLL_MRT, PHASE, SRC, DST>(c, S, D, grid, block, s); break;
+      case VSX_COLL_KBC: launch_bulk<L, VSX_COLL_KBC, PHASE, SRC, DST>(c, S, D, grid, block, s); break;
+      default: launch_bulk<L, VSX_COLL_REG, PHASE, SRC, DST>(c, S, D, grid, block, s); break;
     }
   }
   if constexpr (PHASE == VSX_PHASE_FULL) timer_end(s);
-  if constexpr (PHASE != VSX_PHASE_COLLIDE) {
-    if (c.p.n_walls > 0 && walls_need_edge<L>(c.p)) {
-      const int64_t pw = edge_per_wall<L>(c);
-      const int64_t tot = pw * c.p.n_walls;
-      hipLaunchKernelGGL((k_edge<L, PHASE, SRC, DST>), dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, c, S, D, pw);
-    }
-  }
   VSX_CHECK_LAUNCH();
   return VSX_OK;
 }
