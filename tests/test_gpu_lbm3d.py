@@ -258,3 +258,25 @@ def test_sphere_transpose_is_exact(sim):
         assert np.all(np.diff(lst) > 0)
         assert np.all(I[lst] == k)
     assert np.array_equal(np.sort(slot[:ptr[-1]]), valid)
+
+
+@pytest.mark.parametrize("shape", [(9, 8, 64), (7, 11, 65), (8, 9, 130)])
+@pytest.mark.parametrize("walls", ["two_on_a_face", "three_axes"])
+def test_cells_on_several_walls(sim, shape, walls):
+    """Cells on walls of two and three axes, and a face that carries two walls (the later one wins where it
+    writes), with rows that end at, after and well past a wavefront.  Tolerance: that of the other fused 3D
+    steps (float32 rounding of 12 steps)."""
+    from oracle import lbm3d as O3
+    from oracle import steps as S3
+    W = {"two_on_a_face": [dict(kind="nee", loc="left", ux_wall=0.02), dict(kind="nebb", mode="velocity", loc="front", ux_wall=0.01),
+                           dict(kind="bb", loc="left"), dict(kind="eq", loc="bottom", uz_wall=0.01)],
+         "three_axes": [dict(kind="bb", loc="top", ux_wall=0.03), dict(kind="nee", mode="pressure", loc="right", rho_wall=1.01),
+                        dict(kind="nebb", mode="velocity", loc="back", uy_wall=0.01), dict(kind="nee", loc="left"),
+                        dict(kind="eq", mode="pressure", loc="front", rho_wall=1.0), dict(kind="nee", loc="bottom", uz_wall=0.02)]}[walls]
+    r = np.random.default_rng(5)
+    f0 = (O3.get_equilibrium(1 + 0.02 * r.standard_normal(shape), 0.03 * r.standard_normal((3,) + shape))).astype(np.float32)
+    got = sim.LBM(shape, 1.6, collision="bgk", walls=W).run(dev(f0), 4)
+    ref = f0.astype(np.float64)
+    for _ in range(4):
+        ref = S3.lbm_step3d(ref, 1.6, W, "bgk")
+    assert_close(got, ref, 2e-5, f"{walls} {shape}")

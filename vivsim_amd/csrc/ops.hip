@@ -204,20 +204,11 @@ template <class L>
 __global__ void k_wall(VsxWall w, const float *__restrict__ fpre, const float *f, float *out, Dims d, int64_t nw) {
   const int64_t n = (int64_t)d.n[0] * d.n[1] * d.n[2];
   VSX_GRID_STRIDE(j, nw) {
-    float v[L::Q], fn[L::Q], fp[L::Q];
+    float v[L::Q];
     const int64_t cw = wall_cell<L>(w.loc, j, 0, d);
     load_q<L>(f, n, cw, v);
-    if (wall_needs_neighbor(w)) load_q<L>(f, n, wall_cell<L>(w.loc, j, 1, d), fn);
-    else {
-#pragma unroll
-      for (int i = 0; i < L::Q; ++i) fn[i] = 0.f;
-    }
-    if (wall_needs_pre(w)) load_q<L>(fpre, n, cw, fp);
-    else {
-#pragma unroll
-      for (int i = 0; i < L::Q; ++i) fp[i] = 0.f;
-    }
-    apply_wall<L>(w, j, v, fn, fp);
+    apply_wall<L>(w, j, v, [&](float (&fn)[L::Q]) { load_q<L>(f, n, wall_cell<L>(w.loc, j, 1, d), fn); },
+                  [&](float (&fp)[L::Q]) { load_q<L>(fpre, n, cw, fp); });
     store_q<L>(out, n, cw, v);
   }
 }

@@ -131,16 +131,16 @@ __device__ __noinline__ void wall_state(const StepCtx &c, const typename SRC::T 
     if (J - 1 < c.p.n_walls) {
       const VsxWall &w = c.p.walls[J - 1];
       if (on_wall<L>(c, w.loc, co)) {
-        float fn[L::Q], fp[L::Q];
+        float fn[L::Q];
 #pragma unroll
-        for (int i = 0; i < L::Q; ++i) fn[i] = fp[i] = 0.f;
+        for (int i = 0; i < L::Q; ++i) fn[i] = 0.f;
         if (wall_needs_neighbor(w)) {
           int cn[3];
           inward<L>(w.loc, co, cn);
           wall_state<L, SRC, J - 1, TAG>(c, src, cn, fn);
         }
-        if (wall_needs_pre(w)) local<L, SRC>(c, src, cell_of<L>(c, co[0], co[1], co[2]), fp);
-        apply_wall<L>(w, wall_node<L>(c, w.loc, co), f, fn, fp);
+        apply_wall<L>(w, wall_node<L>(c, w.loc, co), f, Held<L::Q>{fn},
+                      [&](float (&fp)[L::Q]) { local<L, SRC>(c, src, cell_of<L>(c, co[0], co[1], co[2]), fp); });
       }
     }
   }
@@ -193,26 +193,42 @@ __device__ __forceinline__ int wall_class(const StepCtx &c, const int (&co)[3]) 
   return result;
 }
 
-// Populations of a cell of wall class cls >= 0 (the wall location).
+// The wall of a cell of wall class cls >= 0 (the wall location) on its pulled
+// populations.  In 2D the neighbour's loads are issued before anything waits for
+// the cell's own: a second round trip in the wall tiles, the last to start,
+// lengthens a launch (1024^2 VIV step 21.2 -> 22.4 us).  In 3D the registers that
+// this holds cost more.
 template <class L, class SRC>
-__device__ __forceinline__ void single_wall_state(const StepCtx &c, const typename SRC::T *__restrict__ src,
-                                                  const int (&co)[3], int cls, float (&f)[L::Q]) {
-  pull<L, SRC>(c, src, co[0], co[1], co[2], f);
+__device__ __forceinline__ void single_wall(const StepCtx &c, const typename SRC::T *__restrict__ src,
+                                            const int (&co)[3], int cls, float (&f)[L::Q]) {
   static_for<L::n_walls>([&](auto LC) {
     constexpr int LOC = decltype(LC)::value;
     if (LOC != cls) return;
     const VsxWall &w = c.at[LOC];
-    float fn[L::Q], fp[L::Q];
-#pragma unroll
-    for (int i = 0; i < L::Q; ++i) fn[i] = fp[i] = 0.f;
-    if (wall_needs_neighbor(w)) {
+    auto nb = [&](float (&fn)[L::Q]) {
       int cn[3];
       inward<L>(LOC, co, cn);
       pull<L, SRC>(c, src, cn[0], cn[1], cn[2], fn);
+    };
+    auto pre = [&](float (&fp)[L::Q]) { local<L, SRC>(c, src, cell_of<L>(c, co[0], co[1], co[2]), fp); };
+    if constexpr (L::D == 2) {
+      float fn[L::Q];
+#pragma unroll
+      for (int i = 0; i < L::Q; ++i) fn[i] = 0.f;
+      if (wall_needs_neighbor(w)) nb(fn);
+      apply_wall_at<L, LOC>(w, wall_node<L>(c, LOC, co), f, Held<L::Q>{fn}, pre);
+    } else {
+      apply_wall_at<L, LOC>(w, wall_node<L>(c, LOC, co), f, nb, pre);
     }
-    if (wall_needs_pre(w)) local<L, SRC>(c, src, cell_of<L>(c, co[0], co[1], co[2]), fp);
-    apply_wall_at<L, LOC>(w, wall_node<L>(c, LOC, co), f, fn, fp);
   });
+}
+
+// Populations of a cell of wall class cls >= 0.
+template <class L, class SRC>
+__device__ __forceinline__ void single_wall_state(const StepCtx &c, const typename SRC::T *__restrict__ src,
+                                                  const int (&co)[3], int cls, float (&f)[L::Q]) {
+  pull<L, SRC>(c, src, co[0], co[1], co[2], f);
+  single_wall<L, SRC>(c, src, co, cls, f);
 }
 
 // Post-streaming, post-walls populations of any cell.
@@ -440,17 +456,16 @@ __device__ __forceinline__ void edge_cells(const StepCtx &c, const EdgeList &E, 
     const VsxWall &w = c.p.walls[k];
     const int ax = L::w_axis[w.loc], sg = L::w_sign[w.loc];
     const bool on = comp3(s, ax) == sg && !((member >> ax) & 1);
-    float fn[L::Q], fp[L::Q];
+    float fn[L::Q];
 #pragma unroll
-    for (int i = 0; i < L::Q; ++i) fn[i] = fp[i] = 0.f;
+    for (int i = 0; i < L::Q; ++i) fn[i] = 0.f;
     if (wall_needs_neighbor(w)) {
 #pragma unroll
       for (int i = 0; i < L::Q; ++i) fn[i] = __shfl_xor(f[i], 1 << ax, 64);
     }
-    if (on) {
-      if (wall_needs_pre(w)) local<L, SRC>(c, src, cell, fp);
-      apply_wall<L>(w, wall_node<L>(c, w.loc, cn), f, fn, fp);
-    }
+    if (on)
+      apply_wall<L>(w, wall_node<L>(c, w.loc, cn), f, Held<L::Q>{fn},
+                    [&](float (&fp)[L::Q]) { local<L, SRC>(c, src, cell, fp); });
   }
   if (!active || member != 0) return;
   if constexpr (PHASE == VSX_PHASE_FULL) {
@@ -464,8 +479,9 @@ __device__ __forceinline__ void edge_cells(const StepCtx &c, const EdgeList &E, 
 // ------------------------------------------------------------------ kernels
 // Bulk: one thread per cell; blockIdx.x tiles the contiguous axis, blockIdx.y
 // (and z in 3D) the others, so a wavefront touches 64 consecutive cells.
-// EDGE: the first `edge_rows` rows of the outermost grid axis hold the cells on
-// several walls.  Their long chains (a few waves) run beside the bulk, and the
+// k_bulk_walls: walls on several axes; the
+// first `edge_rows` rows of the outermost grid axis hold the cells on several
+// walls.  Their long chains (a few waves) run beside the bulk, and the
 // kernel keeps the register budget of the bulk path (waves_per_eu): what the
 // edge path needs above it is spilled there.
 template <class L>
@@ -496,16 +512,15 @@ __device__ __forceinline__ void bulk_cells(const StepCtx &c, int outer, const ty
     local<L, SRC>(c, src, cell, f);
   } else {
     const int cls = c.p.n_walls > 0 ? wall_class<L>(c, co) : -1;
-    if (cls != -1) {
-      // wall cell: a separate path (own finish and store) keeps the wall code's
-      // register demand out of the interior path below
-      if (cls < 0) return;   // cells on several walls: edge_cells
-      single_wall_state<L, SRC>(c, src, co, cls, f);
-      if constexpr (PHASE != VSX_PHASE_STREAM) finish<L, COLL>(c, cell, co, org, win, f);
-      store_cell<L, DST>(c, dst, cell, f);
-      return;
-    }
+    if (cls < -1) return;   // cells on several walls: edge_cells
     pull<L, SRC>(c, src, co[0], co[1], co[2], f);
+    // A wall across the contiguous axis takes one lane of a row's first or last
+    // wave: the wave runs the wall update for it and goes on together. (With a path
+    // of its own, finish and store included, such a wave did everything twice;
+    // collected in blocks of their own, such lanes read the ends of every row a
+    // second time on another XCD.  20 steps of a 121 x 113 x 127 MRT cavity, where
+    // every wave has such a lane: 2.00, 1.97 and 1.75 ms.)
+    if (cls >= 0) single_wall<L, SRC>(c, src, co, cls, f);
   }
   if constexpr (PHASE != VSX_PHASE_STREAM) finish<L, COLL>(c, cell, co, org, win, f);
   store_cell<L, DST>(c, dst, cell, f);
@@ -520,7 +535,7 @@ __global__ __launch_bounds__(256) void k_bulk(StepCtx c_arg, const typename SRC:
 template <class L, int COLL, int PHASE, class SRC, class DST>
 __global__ __attribute__((amdgpu_flat_work_group_size(64, 256),
                           amdgpu_waves_per_eu(bulk_waves<L>(), bulk_waves<L>()))) void
-k_bulk_edge(StepCtx c_arg, const typename SRC::T *__restrict__ src, typename DST::T *__restrict__ dst, EdgeList E,
+k_bulk_walls(StepCtx c_arg, const typename SRC::T *__restrict__ src, typename DST::T *__restrict__ dst, EdgeList E,
             int edge_rows) {
   const StepCtx &c = kernel_ctx();
   const int outer = L::D == 2 ? blockIdx.y : blockIdx.z;

@@ -99,7 +99,7 @@ void launch_bulk(const StepCtx &c, const typename SRC::T *src, typename DST::T *
       const int64_t per_row = (int64_t)grid.x * (L::D == 2 ? 1 : grid.y);
       const int rows = (int)((blocks + per_row - 1) / per_row);
       (L::D == 2 ? grid.y : grid.z) += rows;
-      hipLaunchKernelGGL((k_bulk_edge<L, COLL, PHASE, SRC, DST>), grid, block, 0, s, c, src, dst, E, rows);
+      hipLaunchKernelGGL((k_bulk_walls<L, COLL, PHASE, SRC, DST>), grid, block, 0, s, c, src, dst, E, rows);
       return;
     }
   }

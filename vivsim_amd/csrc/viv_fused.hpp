@@ -329,21 +329,24 @@ __global__ __launch_bounds__(256) void k_wall_line(StepCtx c_arg, float *__restr
     co[b1] = (int)(j % c.dims[b1]);
   }
   co[a] = L::w_sign[w.loc] > 0 ? 0 : c.dims[a] - 1;
-  float fw[L::Q], fn[L::Q], fp[L::Q];
+  float fw[L::Q];
   const uint32_t cell = cell_of<L>(c, co[0], co[1], co[2]);
+  auto load = [&](uint32_t at, float (&v)[L::Q]) {
 #pragma unroll
-  for (int i = 0; i < L::Q; ++i) {
-    fw[i] = f[(size_t)i * c.n + cell];
-    fn[i] = fp[i] = 0.f;
-  }
-  if (wall_needs_neighbor(w)) {
-    int cn[3];
-    inward<L>(w.loc, co, cn);
-    const uint32_t nb = cell_of<L>(c, cn[0], cn[1], cn[2]);
+    for (int i = 0; i < L::Q; ++i) v[i] = f[(size_t)i * c.n + at];
+  };
+  load(cell, fw);
+  apply_wall<L>(
+      w, wall_node<L>(c, w.loc, co), fw,
+      [&](float (&fn)[L::Q]) {
+        int cn[3];
+        inward<L>(w.loc, co, cn);
+        load(cell_of<L>(c, cn[0], cn[1], cn[2]), fn);
+      },
+      [](float (&fp)[L::Q]) {   // no such wall here (walls_allow_push)
 #pragma unroll
-    for (int i = 0; i < L::Q; ++i) fn[i] = f[(size_t)i * c.n + nb];
-  }
-  apply_wall<L>(w, wall_node<L>(c, w.loc, co), fw, fn, fp);
+        for (int i = 0; i < L::Q; ++i) fp[i] = 0.f;
+      });
 #pragma unroll
   for (int i = 0; i < L::Q; ++i) f[(size_t)i * c.n + cell] = fw[i];
 }
