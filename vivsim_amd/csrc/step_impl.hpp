@@ -138,11 +138,13 @@ int phase_dispatch(const StepCtx &c, const void *src, bool src_f32, void *dst, b
                      : launch_phase<L, VSX_PHASE_COLLIDE, ST, ST>(c, src, dst, s);
     case VSX_PHASE_FULL:
       // an FP32 work buffer larger than the last-level cache: non-temporal
-      // field stores (FP32 only, which keeps the kernel count of the generic
-      // step down; a 16-bit field needs twice the cells to reach that size)
+      // field stores; below it, stores written through (FP32 only, which keeps
+      // the kernel count of the generic step down)
       if constexpr (std::is_same_v<ST, Store<VSX_STORE_F32>>) {
         if ((size_t)c.n * L::Q * sizeof(float) > kLastLevelCacheBytes)
           return launch_phase<L, VSX_PHASE_FULL, ST, Streamed<ST>>(c, src, dst, s);
+        if (write_through(c.n, L::Q, c.dims[L::D - 1], sizeof(float)))
+          return launch_phase<L, VSX_PHASE_FULL, ST, Through<ST>>(c, src, dst, s);
       }
       return launch_phase<L, VSX_PHASE_FULL, ST, ST>(c, src, dst, s);
     case VSX_PHASE_STREAM:

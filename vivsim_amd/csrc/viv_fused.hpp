@@ -390,10 +390,13 @@ inline bool walls_allow_push(const VsxLbm &p) {
 }
 
 // ------------------------------------------------------------------ launches
+// destination storages of the pipelined form only
 template <class B>
-struct IsStreamed : std::false_type {};
+struct PipeOnly : std::false_type {};
 template <class B>
-struct IsStreamed<Streamed<B>> : std::true_type {};
+struct PipeOnly<Streamed<B>> : std::true_type {};
+template <class B>
+struct PipeOnly<Through<B>> : std::true_type {};
 
 Tiles make_tiles(const StepCtx &c);
 
@@ -420,11 +423,11 @@ int launch_fused_p(const StepCtx &c, const VsxIB2D &ib, const void *src, void *d
   if (pipe)
     hipLaunchKernelGGL((k_viv_fused<SRC, DST, COLL, PAIR, MODE, true>), dim3(grid), dim3(kTileCells), lds, s, c, ib,
                        static_cast<const typename SRC::T *>(src), static_cast<typename DST::T *>(dst), step, T);
-  else if constexpr (!IsStreamed<DST>::value)
+  else if constexpr (!PipeOnly<DST>::value)
     hipLaunchKernelGGL((k_viv_fused<SRC, DST, COLL, PAIR, MODE, false>), dim3(1 + grid), dim3(kTileCells), lds, s, c,
                        ib, static_cast<const typename SRC::T *>(src), static_cast<typename DST::T *>(dst), step, T);
   else
-    return fail(VSX_ERR_VALUE, "non-temporal field stores are built for the pipelined form only");
+    return fail(VSX_ERR_VALUE, "these field stores are built for the pipelined form only");
   timer_end(s);
   VSX_CHECK_LAUNCH();
   return VSX_OK;
@@ -434,13 +437,17 @@ template <class SRC, class DST, int COLL, int MODE>
 int launch_fused_c(const StepCtx &c, const VsxIB2D &ib, const void *src, void *dst, int step, hipStream_t s) {
   const Tiles T = make_tiles(c);
   if constexpr (MODE == kModeFull) {
-    // full steps of the pipelined form whose work buffer alone exceeds the
-    // last-level cache: the field stores are non-temporal (such a 16-bit field
-    // has more than kPairMinTiles tiles, so its bulk blocks take tile pairs).
-    // Buffers that exceed the cache only together (2048^2 FP32, 2 x 151 MB)
-    // still gain from plain stores.
+    // full steps of the pipelined form: non-temporal field stores when the work
+    // buffer alone exceeds the last-level cache (such a 16-bit field has more
+    // than kPairMinTiles tiles, so its bulk blocks take tile pairs), written
+    // through below it
     if (ib.fused == 2 && (size_t)c.n * 9 * sizeof(typename DST::T) > kLastLevelCacheBytes)
       return launch_fused_p<SRC, Streamed<DST>, COLL, sizeof(typename SRC::T) == 2, MODE>(c, ib, src, dst, step, s, T);
+  }
+  if constexpr (MODE == kModeFull) {
+    if (ib.fused == 2 && write_through(c.n, 9, c.dims[1], sizeof(typename DST::T)) &&
+        !(sizeof(typename SRC::T) == 2 && T.ntx * T.nty >= kPairMinTiles))
+      return launch_fused_p<SRC, Through<DST>, COLL, false, MODE>(c, ib, src, dst, step, s, T);
   }
   if constexpr (MODE == kModeFull && sizeof(typename SRC::T) == 2) {
     if (T.ntx * T.nty >= kPairMinTiles) return launch_fused_p<SRC, DST, COLL, true, MODE>(c, ib, src, dst, step, s, T);
