@@ -174,6 +174,31 @@ int step_entry(const VsxLbm *p, const void *src, int src_f32, void *dst, int dst
   return step_any<L>(c, src, src_f32 != 0, dst, dst_f32 != 0, phase, as_stream(stream));
 }
 
+// The multi-operation runs (multi2d.hpp), per storage.
+int multi2d_run_f32(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
+int multi2d_run_f16(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
+int multi2d_run_bf16(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
+int multi2d_run_e3m12(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
+
+// Whether a run goes through them: sides that hold the seam and its rings inside
+// a tile, at most one wall per face, and an input that the output of a run of one
+// launch (up to 5 steps) does not overlap.
+inline bool multi2d_takes(const StepCtx &c, const float *f_in, const float *f_out, int n) {
+  for (int l = 0; l < 4; ++l)
+    if (c.order[l] == -2) return false;
+  const int64_t pops = 9 * c.n, gap = f_in < f_out ? f_out - f_in : f_in - f_out;
+  return c.dims[0] >= 40 && c.dims[1] >= 40 && (n > 5 || gap >= pops);
+}
+
+inline int multi2d_run(const StepCtx &c, const float *f_in, float *f_out, void *wa, void *wb, int n, hipStream_t s) {
+  switch (c.p.storage) {
+    case VSX_STORE_F32: return multi2d_run_f32(c, f_in, f_out, wa, wb, n, s);
+    case VSX_STORE_F16S: return multi2d_run_f16(c, f_in, f_out, wa, wb, n, s);
+    case VSX_STORE_BF16S: return multi2d_run_bf16(c, f_in, f_out, wa, wb, n, s);
+    default: return multi2d_run_e3m12(c, f_in, f_out, wa, wb, n, s);
+  }
+}
+
 // n reference steps: COLLIDE(f_in -> a), FULL x (n-1) (a <-> b), STREAM(-> f_out)
 template <class L>
 int run_entry(const VsxLbm *p, const float *f_in, float *f_out, void *wa, void *wb, int n, void *stream) {
@@ -187,6 +212,9 @@ int run_entry(const VsxLbm *p, const float *f_in, float *f_out, void *wa, void *
   if (n == 0) {
     if (f_out != f_in) VSX_HIP(hipMemcpyAsync(f_out, f_in, sizeof(float) * L::Q * c.n, hipMemcpyDeviceToDevice, s));
     return VSX_OK;
+  }
+  if constexpr (L::D == 2) {
+    if (multi2d_takes(c, f_in, f_out, n)) return multi2d_run(c, f_in, f_out, wa, wb, n, s);
   }
   rc = step_any<L>(c, f_in, true, wa, false, VSX_PHASE_COLLIDE, s);
   if (rc) return rc;
