@@ -42,6 +42,9 @@ template <int TX_, int TY_, int KL_, int NT_>
 struct MultiCfg {
   static constexpr int TX = TX_, TY = TY_, KL = KL_, NT = NT_;
   static constexpr int RX = TX + 2 * (KL - 1), RW = TY + 2 * (KL - 1), RC = RX * RW;
+  // waves per SIMD: two workgroups of 768 threads per CU, one of 1024 (whose wall
+  // units then keep their three sets of populations in registers)
+  static constexpr int WAVES = NT > 768 ? 4 : 6;
   // distance of the seam from its tile's edge: the wall cells on both sides of it,
   // their inward neighbours and those neighbours' own lie KL cells and more inside
   static constexpr int SX = KL + 2 > 8 ? 16 : 8, SY = TY >= 64 ? 16 : SX;
@@ -241,7 +244,8 @@ __device__ __forceinline__ void multi_tile(const StepCtx &c, const void *__restr
 }
 
 template <int COLL, class ST, class CF>
-__global__ __attribute__((amdgpu_flat_work_group_size(CF::NT, CF::NT), amdgpu_waves_per_eu(6))) void k_multi2d(StepCtx c_arg, const void *__restrict__ src,
+__global__ __attribute__((amdgpu_flat_work_group_size(CF::NT, CF::NT), amdgpu_waves_per_eu(CF::WAVES))) void
+k_multi2d(StepCtx c_arg, const void *__restrict__ src,
                                                     void *__restrict__ dst, MultiArgs a) {
   const StepCtx &c = kernel_ctx();
   __shared__ typename ST::T lds[9 * CF::RC];
