@@ -200,3 +200,30 @@ def test_batch_split_mode_matches_oracle(sim):
     assert b.clock() == 2 * steps
     for k in range(len(pcs)):
         assert_close(b.view(fa, k), to_np(ref.view(ref_out, k)).astype(np.float64), 1e-5, f"split graph case {k}")
+
+
+@pytest.mark.parametrize("window", [68, 69, 70, 87, 88, 89])
+@pytest.mark.parametrize("markers", [200, 500, 1000])
+def test_batch_launch_modes_by_window(sim, window, markers):
+    """Windows on both sides of the launch modes' limits (both components in LDS up to side 69, one at a time up to
+    88, a launch of its own above) and every lane mapping: the batch gives the case's own run (float32
+    rounding of a few steps where the two kernels' arithmetic is contracted differently)."""
+    D = 30.0
+    pad = (window - int(D)) // 2 if (window - int(D)) % 2 == 0 else None
+    D = D if pad is not None else 31.0
+    pad = pad if pad is not None else (window - 31) // 2
+    c = sim.VIVCase(nx=256, ny=256, D=D, cx=100.0, cy=128.0, n_markers=markers, collision="kbc", forcing="edm", pad=pad)
+    assert c.ib_size == window
+    say(f"batch of two, window {window}, {markers} markers")
+    n = 6
+    b = sim.VIVBatch([c, c], hist_cap=n)
+    b.set_bodies(v=(0.0, 1e-3))
+    got = b.run(b.initial_f(), n)
+    b.check()
+    one = sim.VIV2D(c, pipelined=False, fused=False)
+    one.set_body(v=(0.0, 1e-3))
+    ref, hd, hh = one.run(b.view(b.initial_f(), 0).contiguous(), n)
+    for k in range(2):
+        assert_close(b.view(got, k), to_np(ref).astype(np.float64), 1e-6, f"field {k}")
+        assert_close(b.hist_h[k][:n], to_np(hh), 1e-6, f"force {k}")
+        assert torch.equal(b.view(got, 0), b.view(got, k))

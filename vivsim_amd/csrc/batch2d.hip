@@ -15,11 +15,16 @@
 // step) from device memory, so a captured HIP graph replays correctly: the
 // ready flags, tile counters, body slots and history rows all follow the
 // clock, which each run advances.
-// Split mode (IB windows whose LDS would leave room for only one workgroup
-// per CU, which halves the bulk tiles' occupancy): each step is two
-// launches, the IB workgroups of all cases (k_viv_batch_ib), then the bulk
-// tiles without LDS, which apply the force windows without waiting.
+// The LDS of the IB workgroups is every workgroup's of the launch: two of them per
+// CU need it below half of the CU's (one per CU halves the bulk tiles' occupancy).
+// Windows whose two grid planes exceed that (side 70 to 88) go one component after
+// the other (kModeOne): the IB takes longer, beside the tiles.  16 cases of the
+// sweep's grids (sides 52 and 84), us per step: 58.3, in two launches 79.6.
+// Split mode (larger windows): each step is two launches, the IB workgroups of all
+// cases (k_viv_batch_ib), then the bulk tiles without LDS, which apply the force
+// windows without waiting.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 #include <vector>
@@ -37,17 +42,20 @@ struct BatchCase {
   int32_t hist_cap, band_lo, band_hi, reserved;
 };
 
+// launch modes: one launch per step, two launches, one launch with one-component IB
+constexpr int kModeBoth = 0, kModeSplit = 1, kModeOne = 2;
+
 constexpr int kCaseShift = 20;   // block map entry = case << 20 | tile index
 
 // Populations of one tile cell of case `bc`.  PHASE: COLLIDE reads the
 // caller's post-streaming state in place, FULL / STREAM pull and apply walls.
-template <class SRC, class DST, int COLL, int PHASE, bool SPLIT>
+template <class SRC, class DST, int COLL, int PHASE, int MODE>
 __global__ __attribute__((amdgpu_flat_work_group_size(kTileCells, kTileCells), amdgpu_waves_per_eu(8, 8))) void
 k_viv_batch(const BatchCase *__restrict__ tab, const uint32_t *__restrict__ bmap, int n_cases,
             const typename SRC::T *__restrict__ src, typename DST::T *__restrict__ dst, int step,
             const int32_t *__restrict__ clock) {
   extern __shared__ float lds[];
-  constexpr bool IB = PHASE != VSX_PHASE_STREAM;
+  constexpr bool IB = PHASE != VSX_PHASE_STREAM, SPLIT = MODE == kModeSplit;
   const int b = SPLIT ? (int)blockIdx.x + n_cases : (int)blockIdx.x;   // split: tiles only
   const int gstep = IB ? *clock + step : 0;
   const int slot = gstep & 1;
@@ -70,7 +78,7 @@ k_viv_batch(const BatchCase *__restrict__ tab, const uint32_t *__restrict__ bmap
   }
   if (!SPLIT && b < n_cases) {
     if constexpr (IB && !SPLIT) {
-      ib_atomic<SRC, PHASE == VSX_PHASE_FULL ? kWinPull : kWinLocal, 2, 2, false>(
+      ib_atomic<SRC, PHASE == VSX_PHASE_FULL ? kWinPull : kWinLocal, 2, 2, false, 0, MODE == kModeOne>(
           c, bc.ib, src + bc.f_off, nullptr, gstep < bc.hist_cap ? gstep : -1, gstep, nullptr, bc.ib.body + 6 * slot,
           bc.ib.body + 6 * (slot ^ 1), lds);
       publish_ready(bc.ib, gstep + 1);
@@ -120,9 +128,20 @@ __global__ __launch_bounds__(kIbThreads) void k_viv_batch_ib(const BatchCase *__
                                                           bc.ib.body + 6 * slot, bc.ib.body + 6 * (slot ^ 1), lds);
 }
 
-// Dynamic LDS above which the IB workgroups run in their own launch (two
+// Dynamic LDS above which a workgroup of the launch has a CU for itself (two
 // 1024-thread bulk workgroups per CU need each at most half of the 160 KB).
 constexpr int kBatchSplitLds = 76 * 1024;
+
+// Mode and dynamic LDS of a batch from the LDS of its largest window in both planes.
+int batch_mode(int lds_both, size_t &lds) {
+  lds = lds_both;
+  if (lds_both <= kBatchSplitLds) return kModeBoth;
+  const int S = (int)std::lround(std::sqrt(lds_both / 16.0));   // lds_both = 16 S^2
+  lds = 4 * (size_t)ib_one_lds_words(S);
+  if (lds <= (size_t)kBatchSplitLds) return kModeOne;
+  lds = lds_both;
+  return kModeSplit;
+}
 
 __global__ void k_clock_advance(int32_t *clock, int n) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *clock += n;
@@ -156,15 +175,25 @@ void launch_batch_c(const VsxVivBatch &b, const void *src, void *dst, int step, 
   auto S = static_cast<const typename SRC::T *>(src);
   auto D = static_cast<typename DST::T *>(dst);
   const int32_t *clk = b.clock;
-  if (b.lds_bytes > kBatchSplitLds) {
-    if constexpr (PHASE != VSX_PHASE_STREAM)
-      hipLaunchKernelGGL((k_viv_batch_ib<SRC, PHASE == VSX_PHASE_FULL>), dim3((unsigned)b.n_cases), dim3(kIbThreads),
-                         (size_t)b.lds_bytes, s, tab, S, step, clk);
-    hipLaunchKernelGGL((k_viv_batch<SRC, DST, COLL, PHASE, true>), dim3((unsigned)(b.n_blocks - b.n_cases)),
+  size_t lds = 0;
+  const int mode = batch_mode(b.lds_bytes, lds);
+  if constexpr (PHASE == VSX_PHASE_STREAM) {   // tiles only
+    hipLaunchKernelGGL((k_viv_batch<SRC, DST, COLL, PHASE, kModeSplit>), dim3((unsigned)(b.n_blocks - b.n_cases)),
                        dim3(kTileCells), 0, s, tab, bmap, b.n_cases, S, D, step, clk);
+    return;
   } else {
-    hipLaunchKernelGGL((k_viv_batch<SRC, DST, COLL, PHASE, false>), dim3((unsigned)b.n_blocks), dim3(kTileCells),
-                       (size_t)b.lds_bytes, s, tab, bmap, b.n_cases, S, D, step, clk);
+    if (mode == kModeSplit) {
+      hipLaunchKernelGGL((k_viv_batch_ib<SRC, PHASE == VSX_PHASE_FULL>), dim3((unsigned)b.n_cases), dim3(kIbThreads), lds,
+                         s, tab, S, step, clk);
+      hipLaunchKernelGGL((k_viv_batch<SRC, DST, COLL, PHASE, kModeSplit>), dim3((unsigned)(b.n_blocks - b.n_cases)),
+                         dim3(kTileCells), 0, s, tab, bmap, b.n_cases, S, D, step, clk);
+    } else if (mode == kModeOne) {
+      hipLaunchKernelGGL((k_viv_batch<SRC, DST, COLL, PHASE, kModeOne>), dim3((unsigned)b.n_blocks), dim3(kTileCells), lds,
+                         s, tab, bmap, b.n_cases, S, D, step, clk);
+    } else {
+      hipLaunchKernelGGL((k_viv_batch<SRC, DST, COLL, PHASE, kModeBoth>), dim3((unsigned)b.n_blocks), dim3(kTileCells), lds,
+                         s, tab, bmap, b.n_cases, S, D, step, clk);
+    }
   }
 }
 

@@ -922,11 +922,20 @@ __device__ __forceinline__ void acc_add(float *lds, int SS, int k, float vx, flo
   atomicAdd(&g[k], to_fix(vx));
   atomicAdd(&g[SS + k], to_fix(vy));
 }
+__device__ __forceinline__ void acc_add_one(float *plane, int k, float v) {
+  atomicAdd(&reinterpret_cast<unsigned long long *>(plane)[k], to_fix(v));
+}
+__device__ __forceinline__ float acc_get_one(const float *plane, int k) {
+  return from_fix(reinterpret_cast<const unsigned long long *>(plane)[k]);
+}
 __device__ __forceinline__ float2 acc_get(const float *lds, int SS, int k) {
   const unsigned long long *g = reinterpret_cast<const unsigned long long *>(lds);
   return make_float2(from_fix(g[k]), from_fix(g[SS + k]));
 }
 __host__ __device__ inline int ib_atomic_lds_words(int S) { return 4 * S * S; }
+// One component at a time (ib_atomic with ONE): velocity, over whose start the
+// marks lay, then one plane of the grid in its place; behind it the cell list
+__host__ __device__ inline int ib_one_lds_words(int S) { return 2 * S * S + (S * S + 1) / 2; }
 // SPLIT layout (pipelined IB kernel): velocity, grid, mark array, cell list
 __host__ __device__ inline int ib_split_lds_words(int S) { return 6 * S * S + (S * S + 3) / 4 + (S * S + 1) / 2; }
 
@@ -1039,6 +1048,64 @@ template <bool ACC>
 __device__ __forceinline__ float2 interp_rows(const float *grid, int base, int S, const IbLane &l, const float (&wr)[4],
                                               const float (&wy)[4], bool inside) {
   return inside ? interp_rows<ACC, true>(grid, base, S, l, wr, wy) : interp_rows<ACC, false>(grid, base, S, l, wr, wy);
+}
+
+// One component of the accumulated spread at a marker, from its plane alone: the
+// sums of interp_rows<true>, in their order.
+template <bool INSIDE>
+__device__ __forceinline__ float interp_rows_one(const float *plane, int base, int S, const IbLane &l,
+                                                 const float (&wr)[4], const float (&wy)[4]) {
+  const int SS = S * S;
+  asm volatile("" : "+v"(base));
+  auto fetch = [&](int p) { return acc_get_one(plane, INSIDE ? p : gather_index32(p, SS)); };
+  if (l.tpm == 4) {
+    float v[4], w[4], sx = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[j] = fetch(base + j);
+      w[j] = wr[0] * wy[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sx += w[j] * v[j];
+    float tx = quad_get<0xA0>(sx);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tx += w[j] * v[j];
+    return quad_get<0x55>(tx) + quad_get<0xFF>(tx);
+  }
+  float sx = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i < l.rows) {
+      const int rb = base + i * S;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float v = fetch(rb + j), w = wr[i] * wy[j];
+        sx += w * v;
+      }
+      asm volatile("" : "+v"(sx));
+    }
+  }
+  return marker_sum(sx, l);
+}
+template <bool INSIDE>
+__device__ __forceinline__ void spread_rows_one(float *plane, int base, int S, const IbLane &l, const float (&wr)[4],
+                                                const float (&wy)[4], float fx) {
+  const int SS = S * S;
+  asm volatile("" : "+v"(base));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i < l.rows) {
+      const int rb = base + i * S;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = INSIDE ? rb + j : scatter_index32(rb + j, SS);
+        if (k >= 0) {
+          const float w = wr[i] * wy[j];
+          acc_add_one(plane, k, fx * w);
+        }
+      }
+    }
+  }
 }
 
 // Spread of (fx, fy) over this thread's rows (scatter rule of ib/stencil.py:106-110:
@@ -1163,7 +1230,10 @@ constexpr int kWinLocal = 1;   // read src in place (a post-streaming state)
 constexpr int kWinHalo = 2;    // pull from the FP32 hand-off buffer `halo` [9][S + 4][S + 4] whose origin
                                // is the previous step's window origin - 2 (ib.win_origin[0..1])
 
-template <class SRC, int WSRC, int UW, int TAG, bool SPLIT = false, int TPM = 0>
+// ONE: the two components of the multi-direct forcing one after the other on one
+// plane of the grid (they share the weights only): 10 S^2 instead of 16 S^2 bytes
+// of LDS for a longer loop.
+template <class SRC, int WSRC, int UW, int TAG, bool SPLIT = false, int TPM = 0, bool ONE = false>
 __device__ __forceinline__ void ib_atomic(const StepCtx &c, const VsxIB2D &ib, const typename SRC::T *__restrict__ src,
                                           const float *halo, int hidx, int gstep, int32_t *go_flag,
                                           const double *body_in, double *body_out, float *lds,
@@ -1227,8 +1297,9 @@ __device__ __forceinline__ void ib_atomic(const StepCtx &c, const VsxIB2D &ib, c
   // cell) and the cell list behind the velocity (over the grid's start) or,
   // SPLIT, behind the grid
   float *acc = SPLIT ? lds + 2 * SS : lds;
-  uint8_t *mark = reinterpret_cast<uint8_t *>(lds + (SPLIT ? 6 : 2) * SS);
-  uint16_t *list = reinterpret_cast<uint16_t *>(lds + (SPLIT ? 6 : 2) * SS + (SS + 3) / 4);
+  static_assert(!(SPLIT && ONE), "the pipelined kernel holds both planes");
+  uint8_t *mark = reinterpret_cast<uint8_t *>(lds + (ONE ? 0 : SPLIT ? 6 : 2) * SS);
+  uint16_t *list = reinterpret_cast<uint16_t *>(lds + (SPLIT ? 6 : 2) * SS + (ONE ? 0 : (SS + 3) / 4));
   for (int k = tid; k < (SS + 3) / 4; k += nt) reinterpret_cast<uint32_t *>(mark)[k] = 0u;
   __syncthreads();
   const int x0 = s_org[0], y0 = s_org[1], xc = s_org[2], yc = s_org[3];
@@ -1339,6 +1410,35 @@ __device__ __forceinline__ void ib_atomic(const StepCtx &c, const VsxIB2D &ib, c
   }
   float ubx = ub0x, uby = ub0y, Fx = 0.f, Fy = 0.f;
   const float Ux = (float)s_body[2], Uy = (float)s_body[3];
+  if constexpr (ONE) {
+#pragma unroll 1
+    for (int comp = 0; comp < 2; ++comp) {
+      __syncthreads();   // the velocity, or the plane of x, is dead from here
+      for (int k = tid; k < SS; k += nt) reinterpret_cast<float2 *>(acc)[k] = make_float2(0.f, 0.f);
+      __syncthreads();
+      const float u0 = comp ? ub0y : ub0x, U = comp ? Uy : Ux;
+      float u = u0, F = 0.f;
+      for (int it = 0; it < ib.n_iter; ++it) {
+        const float sf = (U - u) * ds2;
+        F += sf;
+        if (live) {
+          if (inside) spread_rows_one<true>(acc, base, S, l, wr, wy, sf);
+          else spread_rows_one<false>(acc, base, S, l, wr, wy, sf);
+        }
+        __syncthreads();
+        if (it + 1 == ib.n_iter) break;
+        if (live) {
+          const float v = inside ? interp_rows_one<true>(acc, base, S, l, wr, wy)
+                                 : interp_rows_one<false>(acc, base, S, l, wr, wy);
+          u = u0 + 0.5f * v;
+        }
+        __syncthreads();
+      }
+      for (int k = tid; k < SS; k += nt) st_agent(&ib.g_win[comp * SS + k], acc_get_one(acc, k));
+      if (comp) Fy = F;
+      else Fx = F;
+    }
+  } else {
   if constexpr (!SPLIT) {
     __syncthreads();   // the window velocity is dead from here; the grid accumulates the spread force
     for (int k = tid; k < SS; k += nt) reinterpret_cast<float4 *>(acc)[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1366,6 +1466,7 @@ __device__ __forceinline__ void ib_atomic(const StepCtx &c, const VsxIB2D &ib, c
     const float2 g = acc_get(acc, SS, k);
     st_agent(&ib.g_win[k], g.x);
     st_agent(&ib.g_win[SS + k], g.y);
+  }
   }
 
   // body force h = sum(-F) (FP64), one thread per marker
