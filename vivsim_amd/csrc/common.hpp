@@ -64,6 +64,23 @@ inline unsigned grid_for(int64_t n, int block) {
   return (unsigned)g;
 }
 
+// Coordinates of cell c of n in rows of nz cells, planes of ny rows.  In 32 bits
+// where the grid allows: 64-bit divisions by a variable are some 150 instructions
+// each, which the kernels that move a few bytes per cell feel (vorticity of
+// 129 x 97 x 110 cells: 21.9 -> 19.7 us).
+__device__ __forceinline__ void cell_coords(int64_t c, int64_t n, int ny, int nz, int &x, int &y, int &z) {
+  if (n < ((int64_t)1 << 31)) {
+    const uint32_t u = (uint32_t)c, row = u / (uint32_t)nz;
+    z = (int)(u - row * (uint32_t)nz);
+    x = (int)(row / (uint32_t)ny);
+    y = (int)(row - (uint32_t)x * (uint32_t)ny);
+  } else {
+    z = (int)(c % nz);
+    y = (int)((c / nz) % ny);
+    x = (int)(c / ((int64_t)nz * ny));
+  }
+}
+
 // ------------------------------------------------------------------ storage
 // FP32 populations, or 16-bit "shifted" storage of the deviation f_i - s_i
 // from a fixed equilibrium s_i = feq_i(1, u_s) (all arithmetic stays FP32;

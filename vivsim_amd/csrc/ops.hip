@@ -5,6 +5,7 @@
 // thread are strided by n so every wavefront reads 64 consecutive floats per
 // population (coalesced 256-byte segments).
 #include <cstdarg>
+#include <cstdint>
 #include <cstring>
 
 #include "cell.hpp"
@@ -160,9 +161,8 @@ template <class L>
 __global__ void k_stream(const float *__restrict__ f, float *__restrict__ out, int nx, int ny, int nz) {
   const int64_t n = (int64_t)nx * ny * nz;
   VSX_GRID_STRIDE(c, n) {
-    const int z = (int)(c % nz);
-    const int y = (int)((c / nz) % ny);
-    const int x = (int)(c / ((int64_t)nz * ny));
+    int x, y, z;
+    cell_coords(c, n, ny, nz, x, y, z);
 #pragma unroll
     for (int i = 0; i < L::Q; ++i) {
       int xs = x - L::cx[i], ys = y - L::cy[i], zs = z - L::cz[i];
@@ -210,6 +210,33 @@ __global__ void k_wall(VsxWall w, const float *__restrict__ fpre, const float *f
     apply_wall<L>(w, j, v, [&](float (&fn)[L::Q]) { load_q<L>(f, n, wall_cell<L>(w.loc, j, 1, d), fn); },
                   [&](float (&fp)[L::Q]) { load_q<L>(fpre, n, cw, fp); });
     store_q<L>(out, n, cw, v);
+  }
+}
+
+// The same on a copy of a small field in one launch: each thread takes a cell
+// through, the wall's with the wall update.  As a copy and a wall kernel the second
+// adds 4 us (512 x 400 cells: 4.2 + 4.4 us).  Large fields keep those two: the
+// library's copy moves 16 bytes a thread (129 x 97 x 110 cells: 31 + 15 us against 46
+// us; copying around the wall's cells by 16 bytes took 62 us, its index
+// arithmetic bounds it).
+constexpr size_t kWallCopyBytes = size_t(32) << 20;
+
+template <class L>
+__global__ __launch_bounds__(kBlock) void k_wall_copy(VsxWall w, const float *__restrict__ fpre,
+                                                      const float *__restrict__ f, float *__restrict__ out, Dims d) {
+  const int64_t n = (int64_t)d.n[0] * d.n[1] * d.n[2];
+  const int a = L::w_axis[w.loc], face = L::w_sign[w.loc] > 0 ? 0 : d.n[a] - 1;
+  VSX_GRID_STRIDE(c, n) {
+    int x, y, z;
+    cell_coords(c, n, d.n[1], d.n[2], x, y, z);
+    float v[L::Q];
+    load_q<L>(f, n, c, v);
+    if ((a == 0 ? x : (a == 1 ? y : z)) == face) {
+      const int64_t j = a == 0 ? (int64_t)y * d.n[2] + z : (a == 1 ? (int64_t)x * d.n[2] + z : (int64_t)x * d.n[1] + y);
+      apply_wall<L>(w, j, v, [&](float (&fn)[L::Q]) { load_q<L>(f, n, wall_cell<L>(w.loc, j, 1, d), fn); },
+                    [&](float (&fp)[L::Q]) { load_q<L>(fpre, n, c, fp); });
+    }
+    store_q<L>(out, n, c, v);
   }
 }
 
@@ -271,8 +298,15 @@ int boundary(const VsxWall *w, const float *fpre, const float *f, float *out, Di
   VSX_REQUIRE(!wall_needs_pre(*w) || fpre, "bounce-back needs the pre-streaming field");
   const int64_t n = (int64_t)d.n[0] * d.n[1] * d.n[2];
   hipStream_t s = as_stream(stream);
-  if (out != f) VSX_HIP(hipMemcpyAsync(out, f, sizeof(float) * L::Q * n, hipMemcpyDeviceToDevice, s));
   const int64_t nw = wall_nodes<L>(w->loc, d);
+  if (out != f) {
+    if (sizeof(float) * L::Q * n <= kWallCopyBytes) {
+      hipLaunchKernelGGL(k_wall_copy<L>, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, s, *w, fpre, f, out, d);
+      VSX_CHECK_LAUNCH();
+      return VSX_OK;
+    }
+    VSX_HIP(hipMemcpyAsync(out, f, sizeof(float) * L::Q * n, hipMemcpyDeviceToDevice, s));
+  }
   hipLaunchKernelGGL(k_wall<L>, dim3(grid_for(nw, kBlock)), dim3(kBlock), 0, s, *w, fpre, f, out, d, nw);
   VSX_CHECK_LAUNCH();
   return VSX_OK;

@@ -55,7 +55,8 @@ __global__ __launch_bounds__(kPB) void k_post(const float *__restrict__ u, int n
                                               float *__restrict__ out) {
   const int64_t n = (int64_t)nx * ny * nz;
   for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
-    const int z = (int)(c % nz), y = (int)((c / nz) % ny), x = (int)(c / ((int64_t)ny * nz));
+    int x, y, z;
+    cell_coords(c, n, ny, nz, x, y, z);
     if constexpr (OP == VSX_POST_VELOCITY_MAGNITUDE || OP == VSX_POST_KINETIC_ENERGY) {
       float s = 0.f;
 #pragma unroll
@@ -132,7 +133,8 @@ __global__ __launch_bounds__(kPB) void k_mean_partial(const float *__restrict__ 
   const int64_t n = (int64_t)nx * ny * nz;
   double acc = 0.0;
   for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
-    const int z = (int)(c % nz), y = (int)((c / nz) % ny), x = (int)(c / ((int64_t)ny * nz));
+    int x, y, z;
+    cell_coords(c, n, ny, nz, x, y, z);
     float v;
     if constexpr (OP == VSX_POST_KINETIC_ENERGY) {
       float s = 0.f;
