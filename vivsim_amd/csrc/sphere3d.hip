@@ -6,8 +6,11 @@
 //   k_spread3d     A = spread(dF)                                        (cells)
 //   k_mark3d(k)    ub += interp(0.5 A); dF = ...; F += dF                (markers)
 //   ...            (n_iter - 1 times)
-//   k_spread3d     g_win = spread(F); total marker force -F in FP64      (cells)
-//   bulk           collision + forcing with g_win, streaming, walls      (cells)
+//   bulk           g_win = spread(F) by the window's cells, collision + forcing,
+//                  streaming, walls                                      (cells)
+// The total marker force -F of a step is summed in FP64 by a block of the next
+// step's k_win_u3d, or by k_hist3d after the last.  (The last spread was a kernel
+// of its own, 9.4 us with its launch in front of the bulk pass, which hides it.)
 // The body is fixed, so its stencil (computed once, relative to the window
 // origin) is transposed once: spread becomes a gather over the markers that
 // touch each window cell, in ascending marker order -- deterministic and free
@@ -29,8 +32,6 @@
 #include "step_impl.hpp"
 
 namespace vsx {
-
-constexpr int kS3 = 64;   // stencil points per marker (4 x 4 x 4)
 
 struct IB3DDev {
   int32_t *origin;   // [4] window origin (read by the bulk kernel)
@@ -76,26 +77,75 @@ IB3DDev make_dev(const VsxIB3D &ib) {
   return d;
 }
 
-// Window velocity (3 components) of the post-streaming state: pulled from the
-// post-collision state with the walls applied (PULL), or read in place (the
-// first step of a run reads the caller's post-streaming state).
-template <class SRC, bool PULL>
-__global__ __launch_bounds__(256) void k_win_u3d(StepCtx c_arg, IB3DDev d, const typename SRC::T *__restrict__ src) {
+__device__ __forceinline__ double wave_sum3(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// Three consecutive floats as one 12-byte access: the markers' and the window's
+// vectors (u_win, acc: [cells][3]) are gathered, and a gather costs by its requests.
+typedef float vec3 __attribute__((ext_vector_type(3)));
+__device__ __forceinline__ vec3 ld_vec3(const float *p, int64_t k) {
+  typedef float unaligned3 __attribute__((ext_vector_type(3), aligned(4)));
+  return *reinterpret_cast<const unaligned3 *>(p + 3 * k);
+}
+
+// Total marker force sum_m (-F_m) in FP64 (dyn.py:126-136) by a block of 256 threads.
+__device__ __forceinline__ void hist3d(const IB3DDev &d, double *hist) {
+  __shared__ double red[3][4];
+  double h[3] = {0.0, 0.0, 0.0};
+  int m = threadIdx.x;
+  for (; m + 3 * 256 < d.M; m += 4 * 256) {   // four markers' loads in flight
+    vec3 F[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) F[u] = ld_vec3(d.F, m + 256 * u);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      for (int a = 0; a < 3; ++a) h[a] -= (double)F[u][a];
+  }
+  for (; m < d.M; m += 256)
+    for (int a = 0; a < 3; ++a) h[a] -= (double)d.F[3 * m + a];
+  for (int a = 0; a < 3; ++a) h[a] = wave_sum3(h[a]);
+  if ((threadIdx.x & 63) == 0)
+    for (int a = 0; a < 3; ++a) red[a][threadIdx.x >> 6] = h[a];
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int a = 0; a < 3; ++a) hist[a] = red[a][0] + red[a][1] + red[a][2] + red[a][3];
+}
+__global__ __launch_bounds__(256) void k_hist3d(IB3DDev d, double *hist) { hist3d(d, hist); }
+
+// Window velocity (3 components) of the post-streaming state: read in place
+// (kWinHere: the first step of a run reads the caller's post-streaming state) or
+// pulled from the post-collision state, with the walls applied when the window
+// touches a walled face (kWinWalls; the wall code's registers and scratch memory
+// make that kernel 7.0 us instead of 5.3 at a 32^3 window).  With hist_prev, the
+// last block writes the previous step's total marker force.
+constexpr int kWinHere = 0, kWinClear = 1, kWinWalls = 2;
+template <class SRC, int MODE>
+__global__ __launch_bounds__(256) void k_win_u3d(StepCtx c_arg, IB3DDev d, const typename SRC::T *__restrict__ src,
+                                                 double *hist_prev) {
   const StepCtx &c = kernel_ctx();
+  if (hist_prev && blockIdx.x == gridDim.x - 1) {
+    hist3d(d, hist_prev);
+    return;
+  }
   const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (k == 0) {
     for (int a = 0; a < 3; ++a) d.origin[a] = d.org[a];
   }
   if (k >= d.cells) return;
-  const int r2 = (int)(k % d.S[2]);
-  const int r1 = (int)((k / d.S[2]) % d.S[1]);
-  const int r0 = (int)(k / ((int64_t)d.S[2] * d.S[1]));
+  const uint32_t row = (uint32_t)k / (uint32_t)d.S[2];   // (fewer than 2^31 cells)
+  const int r2 = (int)((uint32_t)k % (uint32_t)d.S[2]);
+  const int r1 = (int)(row % (uint32_t)d.S[1]);
+  const int r0 = (int)(row / (uint32_t)d.S[1]);
   const int co[3] = {d.org[0] + r0, d.org[1] + r1, d.org[2] + r2};
   float f[19], rho, u[3];
-  if constexpr (PULL) cell_state<D3Q19, SRC>(c, src, co, f);
+  if constexpr (MODE == kWinWalls) cell_state<D3Q19, SRC>(c, src, co, f);
+  else if constexpr (MODE == kWinClear) pull<D3Q19, SRC>(c, src, co[0], co[1], co[2], f);
   else local<D3Q19, SRC>(c, src, cell_of<D3Q19>(c, co[0], co[1], co[2]), f);
   macroscopic<D3Q19>(f, rho, u);
-  for (int a = 0; a < 3; ++a) d.u_win[a * d.cells + k] = u[a];
+  for (int a = 0; a < 3; ++a) d.u_win[3 * k + a] = u[a];
 }
 
 // Marker phase `it` of the multi-direct forcing loop (ib/mdf.py:45-57).
@@ -112,7 +162,8 @@ __global__ __launch_bounds__(256) void k_mark3d(IB3DDev d, int it) {
   const float *grid = it == 0 ? d.u_win : d.acc;
   const int64_t gi = gather_index(d.I[(int64_t)m * kS3 + lane], d.cells);
   const float w = d.W[(int64_t)m * kS3 + lane];
-  float v0 = grid[gi], v1 = grid[d.cells + gi], v2 = grid[2 * d.cells + gi];
+  const vec3 v = ld_vec3(grid, gi);
+  float v0 = v.x, v1 = v.y, v2 = v.z;
   if (it != 0) {
     v0 *= 0.5f;
     v1 *= 0.5f;
@@ -148,64 +199,70 @@ __global__ __launch_bounds__(256) void k_mark3d(IB3DDev d, int it) {
   }
 }
 
-__device__ __forceinline__ double wave_sum3(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
 // out[a][k] = sum over the stencil slots that land on window cell k of
-// mf[m][a] * W[slot] (ib/stencil.py:81-110 as a gather).  With hist, block 0
-// also writes the total marker force sum_m (-F_m) in FP64 (dyn.py:126-136).
+// mf[m][a] * W[slot] (ib/stencil.py:81-110 as a gather), in slot order.  Eight lanes
+// per cell: each loads every eighth slot of the list, eight in flight, and the
+// group then adds them up in order, lane after lane.  agent: into planes, else [cells][3].  (A thread per cell walks its
+// list of up to some 60 slots in dependent round trips: 9.4 us at 4096 markers,
+// 7.4 so.)
+template <int I>
+__device__ __forceinline__ float group8_get(float v) {   // lane I of each group of eight
+  return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (I << 5) | 0x18));
+}
 __global__ __launch_bounds__(256) void k_spread3d(IB3DDev d, const float *__restrict__ mf, float *__restrict__ out,
-                                                  double *hist, bool agent) {
-  const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (k < d.cells) {
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f;
-    const int e1 = d.cell_ptr[k + 1];
-    int e = d.cell_ptr[k];
-    for (; e + 4 <= e1; e += 4) {   // four slots' loads in flight, summed in slot order
-      int slot[4];
+                                                  bool agent) {
+  const int64_t k = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 3;
+  const int i = threadIdx.x & 7;
+  if (k - ((threadIdx.x & 63) >> 3) >= d.cells) return;   // whole wavefronts
+  const bool on = k < d.cells;
+  int e = on ? d.cell_ptr[k] : 0;
+  const int e1 = on ? d.cell_ptr[k + 1] : 0;
+  float s0 = 0.f, s1 = 0.f, s2 = 0.f;
+  while (__any(e < e1)) {
+    int slot[8];
+    float w[8];
+    vec3 f[8];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) slot[u] = d.cell_slot[e + u];
+    for (int j = 0; j < 8; ++j) {
+      const int q = e + 8 * j + i;
+      slot[j] = q < e1 ? d.cell_slot[q] : -1;
+    }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int m = slot[u] / kS3;
-        const float w = d.W[slot[u]];
-        s0 += mf[3 * m] * w;
-        s1 += mf[3 * m + 1] * w;
-        s2 += mf[3 * m + 2] * w;
+    for (int j = 0; j < 8; ++j) {
+      if (slot[j] >= 0) {
+        w[j] = d.W[slot[j]];
+        f[j] = ld_vec3(mf, slot[j] / kS3);
+      } else {
+        w[j] = 0.f;
+        f[j] = vec3{0.f, 0.f, 0.f};
       }
     }
-    for (; e < e1; ++e) {
-      const int slot = d.cell_slot[e];
-      const int m = slot / kS3;
-      const float w = d.W[slot];
-      s0 += mf[3 * m] * w;
-      s1 += mf[3 * m + 1] * w;
-      s2 += mf[3 * m + 2] * w;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (!__any(e + 8 * j < e1)) break;
+      static_for<8>([&](auto IC) {
+        constexpr int I = decltype(IC)::value;
+        const float ww = group8_get<I>(w[j]);
+        const float a0 = group8_get<I>(f[j].x), a1 = group8_get<I>(f[j].y), a2 = group8_get<I>(f[j].z);
+        if (e + 8 * j + I < e1) {
+          s0 += a0 * ww;
+          s1 += a1 * ww;
+          s2 += a2 * ww;
+        }
+      });
     }
-    if (agent) {   // read by the bulk pass of another stream
+    e += 64;
+  }
+  if (on && i == 0) {
+    if (agent) {   // the force window, read by the bulk pass of another stream
       st_agent(&out[k], s0);
       st_agent(&out[d.cells + k], s1);
       st_agent(&out[2 * d.cells + k], s2);
     } else {
-      out[k] = s0;
-      out[d.cells + k] = s1;
-      out[2 * d.cells + k] = s2;
+      out[3 * k] = s0;
+      out[3 * k + 1] = s1;
+      out[3 * k + 2] = s2;
     }
-  }
-  if (hist && blockIdx.x == 0) {
-    __shared__ double red[3][4];
-    double h[3] = {0.0, 0.0, 0.0};
-    for (int m = threadIdx.x; m < d.M; m += blockDim.x)
-      for (int a = 0; a < 3; ++a) h[a] -= (double)d.F[3 * m + a];
-    for (int a = 0; a < 3; ++a) h[a] = wave_sum3(h[a]);
-    if ((threadIdx.x & 63) == 0)
-      for (int a = 0; a < 3; ++a) red[a][threadIdx.x >> 6] = h[a];
-    __syncthreads();
-    if (threadIdx.x == 0)
-      for (int a = 0; a < 3; ++a) hist[a] = red[a][0] + red[a][1] + red[a][2] + red[a][3];
   }
 }
 
@@ -240,7 +297,7 @@ __global__ __launch_bounds__(256) void k_win_u3d_halo(IB3DDev d, const float *__
   for (int q = 0; q < 19; ++q)
     f[q] = ld_agent(&h[q * EE + ((int64_t)(r0 - D3Q19::cx[q]) * E1 + (r1 - D3Q19::cy[q])) * E2 + (r2 - D3Q19::cz[q])]);
   macroscopic<D3Q19>(f, rho, u);
-  for (int a = 0; a < 3; ++a) d.u_win[a * d.cells + k] = u[a];
+  for (int a = 0; a < 3; ++a) d.u_win[3 * k + a] = u[a];
 }
 
 // ready flag of step `step`: the force window (written with st_agent by the
@@ -391,37 +448,59 @@ __global__ void k_sort_lists(const int32_t *ptr, int64_t n_grid, int32_t *slot) 
 
 // ------------------------------------------------------------------ host side
 
-template <class SRC, bool PULL>
-void launch_win_u(const StepCtx &c, const IB3DDev &d, const void *src, hipStream_t s) {
-  hipLaunchKernelGGL((k_win_u3d<SRC, PULL>), dim3((unsigned)((d.cells + 255) / 256)), dim3(256), 0, s, c, d,
-                     static_cast<const typename SRC::T *>(src));
+// whether a window cell lies on a wall
+bool window_on_wall(const StepCtx &c, const IB3DDev &d) {
+  for (int l = 0; l < 6; ++l) {
+    const int a = D3Q19::w_axis[l];
+    if (c.order[l] != -1 && (D3Q19::w_sign[l] > 0 ? d.org[a] == 0 : d.org[a] + d.S[a] == c.dims[a])) return true;
+  }
+  return false;
 }
 
-void win_u_any(const StepCtx &c, const IB3DDev &d, const void *src, bool first, hipStream_t s) {
-  if (first) return launch_win_u<Store<VSX_STORE_F32>, false>(c, d, src, s);
+template <class SRC>
+void launch_win_u(const StepCtx &c, const IB3DDev &d, const void *src, bool first, double *hist_prev, hipStream_t s) {
+  const dim3 grid((unsigned)((d.cells + 255) / 256 + (hist_prev ? 1 : 0)));
+  auto S = static_cast<const typename SRC::T *>(src);
+  if constexpr (std::is_same_v<SRC, Store<VSX_STORE_F32>>) {
+    if (first) {
+      hipLaunchKernelGGL((k_win_u3d<SRC, kWinHere>), grid, dim3(256), 0, s, c, d, S, hist_prev);
+      return;
+    }
+  }
+  if (window_on_wall(c, d)) hipLaunchKernelGGL((k_win_u3d<SRC, kWinWalls>), grid, dim3(256), 0, s, c, d, S, hist_prev);
+  else hipLaunchKernelGGL((k_win_u3d<SRC, kWinClear>), grid, dim3(256), 0, s, c, d, S, hist_prev);
+}
+
+void win_u_any(const StepCtx &c, const IB3DDev &d, const void *src, bool first, double *hist_prev, hipStream_t s) {
+  if (first) return launch_win_u<Store<VSX_STORE_F32>>(c, d, src, true, hist_prev, s);
   switch (c.p.storage) {
-    case VSX_STORE_F32: return launch_win_u<Store<VSX_STORE_F32>, true>(c, d, src, s);
-    case VSX_STORE_F16S: return launch_win_u<Store<VSX_STORE_F16S>, true>(c, d, src, s);
-    case VSX_STORE_BF16S: return launch_win_u<Store<VSX_STORE_BF16S>, true>(c, d, src, s);
-    default: return launch_win_u<Store<VSX_STORE_E3M12S>, true>(c, d, src, s);
+    case VSX_STORE_F32: return launch_win_u<Store<VSX_STORE_F32>>(c, d, src, false, hist_prev, s);
+    case VSX_STORE_F16S: return launch_win_u<Store<VSX_STORE_F16S>>(c, d, src, false, hist_prev, s);
+    case VSX_STORE_BF16S: return launch_win_u<Store<VSX_STORE_BF16S>>(c, d, src, false, hist_prev, s);
+    default: return launch_win_u<Store<VSX_STORE_E3M12S>>(c, d, src, false, hist_prev, s);
   }
 }
 
-// The IB of one step.  pipe_step >= 0 (pipelined form): the window velocity of a
-// step after the first comes from the hand-off buffer, the force window is
-// written with st_agent and the ready flag raised for step pipe_step.
-int ib3d_phase(const StepCtx &c, const IB3DDev &d, const void *src, bool first, double *hist, hipStream_t s,
-               const float *halo = nullptr, int pipe_step = -1) {
+// The IB of one step up to the marker forces.  hist_prev: see k_win_u3d.
+// pipe_step >= 0 (pipelined form): the window velocity of a step after the first
+// comes from the hand-off buffer, the force window is written with st_agent, this
+// step's total force into hist, and the ready flag raised for step pipe_step.
+int ib3d_phase(const StepCtx &c, const IB3DDev &d, const void *src, bool first, double *hist_prev, hipStream_t s,
+               const float *halo = nullptr, int pipe_step = -1, double *hist = nullptr) {
   const unsigned gm = (unsigned)((d.M + 3) / 4), gc = (unsigned)((d.cells + 255) / 256);   // k_mark3d: 4 markers / block
+  const unsigned gs = (unsigned)((8 * d.cells + 255) / 256);                               // k_spread3d: 8 lanes / cell
   if (pipe_step > 0 && !first) hipLaunchKernelGGL(k_win_u3d_halo, dim3(gc), dim3(256), 0, s, d, halo, pipe_step);
-  else win_u_any(c, d, src, first, s);
+  else win_u_any(c, d, src, first, hist_prev, s);
   hipLaunchKernelGGL(k_mark3d, dim3(gm), dim3(256), 0, s, d, 0);
   for (int it = 1; it < d.n_iter; ++it) {
-    hipLaunchKernelGGL(k_spread3d, dim3(gc), dim3(256), 0, s, d, (const float *)d.dF, d.acc, (double *)nullptr, false);
+    hipLaunchKernelGGL(k_spread3d, dim3(gs), dim3(256), 0, s, d, (const float *)d.dF, d.acc, false);
     hipLaunchKernelGGL(k_mark3d, dim3(gm), dim3(256), 0, s, d, it);
   }
-  hipLaunchKernelGGL(k_spread3d, dim3(gc), dim3(256), 0, s, d, (const float *)d.F, d.g_win, hist, pipe_step >= 0);
-  if (pipe_step >= 0) hipLaunchKernelGGL(k_publish3d, dim3(1), dim3(1), 0, s, d, pipe_step);
+  if (pipe_step >= 0) {
+    hipLaunchKernelGGL(k_spread3d, dim3(gs), dim3(256), 0, s, d, (const float *)d.F, d.g_win, true);
+    if (hist) hipLaunchKernelGGL(k_hist3d, dim3(1), dim3(256), 0, s, d, hist);
+    hipLaunchKernelGGL(k_publish3d, dim3(1), dim3(1), 0, s, d, pipe_step);
+  }
   VSX_CHECK_LAUNCH();
   return VSX_OK;
 }
@@ -515,7 +594,7 @@ int sphere_run(const VsxLbm *p, const VsxIB3D *ib, const float *f_in, float *f_o
     VSX_HIP(hipStreamWaitEvent(r->s, r->fork, 0));
     VSX_HIP(hipStreamWaitEvent(r->b, r->fork, 0));
     for (int t = 0; t < n; ++t) {
-      rc = ib3d_phase(c, d, f_in, t == 0, ib->hist_h ? ib->hist_h + 3 * (int64_t)t : nullptr, r->s, ib->halo, t);
+      rc = ib3d_phase(c, d, f_in, t == 0, nullptr, r->s, ib->halo, t, ib->hist_h ? ib->hist_h + 3 * (int64_t)t : nullptr);
       if (rc) return rc;
       void *dst = bufs[t & 1];
       switch (c.p.storage) {
@@ -534,14 +613,21 @@ int sphere_run(const VsxLbm *p, const VsxIB3D *ib, const float *f_in, float *f_o
     const StepCtx cs = make_ctx<D3Q19>(*p, Window{nullptr, nullptr, {0, 0, 0}});
     return step_any<D3Q19>(cs, cur, false, f_out, true, VSX_PHASE_STREAM, s);
   }
+  // the window's cells gather their force from the markers' in the bulk pass
+  StepCtx cb = c;
+  cb.win.F = d.F;
+  cb.win.W = d.W;
+  cb.win.cell_ptr = d.cell_ptr;
+  cb.win.cell_slot = d.cell_slot;
   for (int t = 0; t < n; ++t) {
     void *dst = bufs[t & 1];
-    rc = ib3d_phase(c, d, cur, t == 0, ib->hist_h ? ib->hist_h + 3 * (int64_t)t : nullptr, s);
+    rc = ib3d_phase(c, d, cur, t == 0, ib->hist_h && t > 0 ? ib->hist_h + 3 * (int64_t)(t - 1) : nullptr, s);
     if (rc) return rc;
-    rc = step_any<D3Q19>(c, cur, t == 0, dst, false, t == 0 ? VSX_PHASE_COLLIDE : VSX_PHASE_FULL, s);
+    rc = step_any<D3Q19>(cb, cur, t == 0, dst, false, t == 0 ? VSX_PHASE_COLLIDE : VSX_PHASE_FULL, s);
     if (rc) return rc;
     cur = dst;
   }
+  if (ib->hist_h) hipLaunchKernelGGL(k_hist3d, dim3(1), dim3(256), 0, s, d, ib->hist_h + 3 * (int64_t)(n - 1));
   const StepCtx cs = make_ctx<D3Q19>(*p, Window{nullptr, nullptr, {0, 0, 0}});
   return step_any<D3Q19>(cs, cur, false, f_out, true, VSX_PHASE_STREAM, s);
 }

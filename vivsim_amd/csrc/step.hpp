@@ -37,7 +37,42 @@ struct Window {
   const int32_t *origin;   // [3] clamped window origin, or null (no window)
   const float *g;          // [D][S0][S1(][S2)]
   int32_t size[3];
+  // 3D: the forces `F` [M][3] of the markers, gathered by the window's cells
+  // themselves (null: read from g); stencil weights and cell -> slot lists of
+  // vsx_ib3d_transpose_stencil, `points` slots per marker; also stored in g
+  const float *F = nullptr, *W = nullptr;
+  const int32_t *cell_ptr = nullptr, *cell_slot = nullptr;
 };
+
+// Sum over the stencil slots that land on window cell k of mf[m][a] * W[slot]
+// (ib/stencil.py:81-110 as a gather), in slot order.
+constexpr int kS3 = 64;   // stencil points per marker (4 x 4 x 4)
+__device__ __forceinline__ void gather_cell3(const float *__restrict__ mf, const float *__restrict__ W,
+                                             const int32_t *__restrict__ cell_ptr,
+                                             const int32_t *__restrict__ cell_slot, int64_t k, float (&s)[3]) {
+  s[0] = s[1] = s[2] = 0.f;
+  const int e1 = cell_ptr[k + 1];
+  int e = cell_ptr[k];
+  for (; e + 4 <= e1; e += 4) {   // four slots' loads in flight, summed in slot order
+    int slot[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) slot[u] = cell_slot[e + u];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int m = slot[u] / kS3;
+      const float w = W[slot[u]];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) s[a] += mf[3 * m + a] * w;
+    }
+  }
+  for (; e < e1; ++e) {
+    const int slot = cell_slot[e];
+    const int m = slot / kS3;
+    const float w = W[slot];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) s[a] += mf[3 * m + a] * w;
+  }
+}
 
 struct StepCtx {
   VsxLbm p;
@@ -275,6 +310,18 @@ __device__ __forceinline__ void body_force(const StepCtx &c, uint32_t cell, cons
 #pragma unroll
       for (int a = 1; a < L::D; ++a) k = k * c.win.size[a] + r[a];
       const int wn = c.win.size[0] * c.win.size[1] * (L::D == 3 ? c.win.size[2] : 1);
+      if constexpr (L::D == 3) {
+        if (c.win.F) {
+          float s[3];
+          gather_cell3(c.win.F, c.win.W, c.win.cell_ptr, c.win.cell_slot, k, s);
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            const_cast<float *>(c.win.g)[a * wn + k] = s[a];
+            g[a] += s[a];
+          }
+          return;
+        }
+      }
 #pragma unroll
       for (int a = 0; a < L::D; ++a) {
         // 2D: the force window may come from the IB workgroup of this launch;
