@@ -64,16 +64,11 @@ k_viv_batch(const BatchCase *__restrict__ tab, const uint32_t *__restrict__ bmap
   int org[3] = {0, 0, 0};
   int wx0 = 0, wx1 = -1, wy0 = 0, wy1 = -1;
   if constexpr (IB) {
-    __shared__ int s_org[2];
-    if (threadIdx.x == 0) {
-      int o[4];
-      window_origin(c, bc.ib, bc.ib.body + 6 * slot, o);
-      s_org[0] = o[2];
-      s_org[1] = o[3];
-    }
-    __syncthreads();
-    org[0] = s_org[0];
-    org[1] = s_org[1];
+    // every wave for itself, as in k_viv_fused
+    int o[4];
+    window_origin(c, bc.ib, bc.ib.body + 6 * slot, o);
+    org[0] = __builtin_amdgcn_readfirstlane(o[2]);
+    org[1] = __builtin_amdgcn_readfirstlane(o[3]);
     window_tiles(bc.T, org[0], org[1], bc.ib.win, wx0, wx1, wy0, wy1);
   }
   if (!SPLIT && b < n_cases) {
