@@ -104,7 +104,7 @@ k_viv_batch(const BatchCase *__restrict__ tab, const uint32_t *__restrict__ bmap
     if (win) wait_ready(bc.ib, gstep + 1);
   }
   if (!valid) return;
-  if constexpr (PHASE != VSX_PHASE_STREAM) finish<D2Q9, COLL>(c, cell, co, org, win, f);
+  if constexpr (PHASE != VSX_PHASE_STREAM) finish<D2Q9, COLL, PHASE == VSX_PHASE_COLLIDE>(c, cell, co, org, win, f);
   store_cell<D2Q9, DST>(c, d_case, cell, f);
 }
 

@@ -374,8 +374,13 @@ __device__ __forceinline__ void mrt_d3q19(float (&f)[19], const float (&feq)[19]
   for (int i = 0; i < 19; ++i) d[i] = feq[i] - f[i];
 #pragma unroll
   for (int k = 0; k < 19; ++k) {
-    float v = rates[k] * mrow3(k, d);
-    if (HAS_F) v += (1.f - 0.5f * rates[k]) * mrow3(k, F);
+    // one rounding of the relaxed moment, not a fused one for each sum it enters
+    float v;
+    {
+#pragma clang fp contract(off)
+      v = rates[k] * mrow3(k, d);
+    }
+    if (HAS_F) v = __builtin_fmaf(1.f - 0.5f * rates[k], mrow3(k, F), v);
     r[k] = v;
   }
 #pragma unroll

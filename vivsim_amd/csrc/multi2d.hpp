@@ -165,7 +165,8 @@ __device__ __forceinline__ void multi_tile(const StepCtx &c, const void *__restr
     };
     auto emit = [&](const int (&co)[3], int l, float (&f)[9]) {
       const uint32_t cell = (uint32_t)co[0] * ny + co[1];
-      if (collide) finish<D2Q9, COLL>(c, cell, co, org, false, f);
+      if (COLL == VSX_COLL_BGK && in_place) finish<D2Q9, COLL, true>(c, cell, co, org, false, f);
+      else if (collide) finish<D2Q9, COLL>(c, cell, co, org, false, f);
       if (s < a.k) lds_put<ST, CF>(c, lds, s, l, f);
       else if (a.last) store_cell<D2Q9, F32>(c, static_cast<float *>(dst), cell, f);
       else if (a.store == 1) store_cell<D2Q9, Streamed<ST>>(c, static_cast<T *>(dst), cell, f);

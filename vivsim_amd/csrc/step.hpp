@@ -346,7 +346,10 @@ __device__ __forceinline__ bool window_origin_of(const StepCtx &c, int (&org)[3]
 // collision + forcing of one cell, composed as in the reference examples:
 //   Guo: u* = u + g / (2 rho) in the equilibrium and the forcing term (poiseuille_channel.py:99-128)
 //   EDM: uncorrected u, f += F(g, u)                               (poiseuille_channel.py:84-97)
-template <class L, int COLL>
+// Which of BGK's two products is rounded is written out (IN_PLACE: the unforced
+// collision that opens a run): left to the compiler it depends on the code around,
+// and kernels that run the same operation then differ in the last bit.
+template <class L, int COLL, bool IN_PLACE = false>
 __device__ __forceinline__ void collide_force(float (&f)[L::Q], float rho, const float (&u)[3], const float (&g)[3],
                                               int forcing, float omega, const float *rates) {
   const bool has_g = forcing != VSX_FORCE_NONE && (g[0] != 0.f || g[1] != 0.f || g[2] != 0.f);
@@ -368,7 +371,8 @@ __device__ __forceinline__ void collide_force(float (&f)[L::Q], float rho, const
   if constexpr (COLL == VSX_COLL_BGK) {
     const float a = 1.f - omega;
 #pragma unroll
-    for (int i = 0; i < L::Q; ++i) f[i] = a * f[i] + omega * feq[i];
+    for (int i = 0; i < L::Q; ++i)
+      f[i] = IN_PLACE ? __builtin_fmaf(omega, feq[i], a * f[i]) : __builtin_fmaf(a, f[i], omega * feq[i]);
   } else if constexpr (COLL == VSX_COLL_KBC) {
     if constexpr (L::Q == 9) kbc_d2q9(f, feq, omega);
     else kbc_d3q19<L>(f, feq, omega);
@@ -408,7 +412,7 @@ __device__ __forceinline__ void store_cell(const StepCtx &c, typename DST::T *__
 
 // finish() of a cell that carries no body force (no g field, no uniform g, not
 // in the IB window): the forced branches are compiled out.
-template <class L, int COLL>
+template <class L, int COLL, bool IN_PLACE = false>
 __device__ __forceinline__ void finish_unforced(const StepCtx &c, float (&f)[L::Q]) {
   float rho, u[3];
   macroscopic<L>(f, rho, u);
@@ -419,18 +423,18 @@ __device__ __forceinline__ void finish_unforced(const StepCtx &c, float (&f)[L::
     mrt_d2q9_unforced(f, rho, u, r);
   } else {
     const float g[3] = {0.f, 0.f, 0.f};
-    collide_force<L, COLL>(f, rho, u, g, VSX_FORCE_NONE, c.p.omega, c.p.mrt_rates);
+    collide_force<L, COLL, IN_PLACE>(f, rho, u, g, VSX_FORCE_NONE, c.p.omega, c.p.mrt_rates);
   }
 }
 
-template <class L, int COLL>
+template <class L, int COLL, bool IN_PLACE = false>
 __device__ __forceinline__ void finish(const StepCtx &c, uint32_t cell, const int (&co)[3], const int (&org)[3],
                                        bool win, float (&f)[L::Q]) {
   bool unforced = !win && !c.p.g;
 #pragma unroll
   for (int a = 0; a < L::D; ++a) unforced = unforced && c.p.g_uniform[a] == 0.f;
   if (unforced) {
-    finish_unforced<L, COLL>(c, f);
+    finish_unforced<L, COLL, IN_PLACE>(c, f);
     return;
   }
   float rho, u[3], g[3];
@@ -569,7 +573,7 @@ __device__ __forceinline__ void bulk_cells(const StepCtx &c, int outer, const ty
     // every wave has such a lane: 2.00, 1.97 and 1.75 ms.)
     if (cls >= 0) single_wall<L, SRC>(c, src, co, cls, f);
   }
-  if constexpr (PHASE != VSX_PHASE_STREAM) finish<L, COLL>(c, cell, co, org, win, f);
+  if constexpr (PHASE != VSX_PHASE_STREAM) finish<L, COLL, PHASE == VSX_PHASE_COLLIDE>(c, cell, co, org, win, f);
   store_cell<L, DST>(c, dst, cell, f);
 }
 

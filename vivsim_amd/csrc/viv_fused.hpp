@@ -121,7 +121,7 @@ __device__ __forceinline__ void bulk_cell(const StepCtx &c, const typename SRC::
                                           typename DST::T *__restrict__ dst, const int (&co)[3], const int (&org)[3]) {
   float f[9];
   tile_cell_state<SRC, MODE>(c, src, co, f);
-  finish<D2Q9, COLL>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, false, f);
+  finish<D2Q9, COLL, MODE == kModeFirst>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, false, f);
   tile_store<DST, MODE>(c, dst, co, f);
 }
 
@@ -223,7 +223,7 @@ k_viv_fused(StepCtx c_arg, VsxIB2D ib, const typename SRC::T *__restrict__ src, 
     if (valid) tile_cell_state<SRC, MODE>(c, src, co, f);
     if (force) wait_ready(ib, gstep + 1);
     if (valid) {
-      finish<D2Q9, COLL>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, force, f);
+      finish<D2Q9, COLL, MODE == kModeFirst>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, force, f);
       tile_store<DST, MODE>(c, dst, co, f);
     }
     if constexpr (MODE != kModeLast) {
@@ -244,7 +244,7 @@ k_viv_fused(StepCtx c_arg, VsxIB2D ib, const typename SRC::T *__restrict__ src, 
     if (valid) tile_cell_state<SRC, MODE>(c, src, co, f);
     wait_ready(ib, gstep + 1);
     if (!valid) return;
-    finish<D2Q9, COLL>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, true, f);
+    finish<D2Q9, COLL, MODE == kModeFirst>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, true, f);
     tile_store<DST, MODE>(c, dst, co, f);
     return;
   }
@@ -259,7 +259,7 @@ k_viv_fused(StepCtx c_arg, VsxIB2D ib, const typename SRC::T *__restrict__ src, 
     if (cls >= 0) {
       // wall cell: own path, keeping the wall code's registers out of the interior path
       single_wall_state<D2Q9, SRC>(c, src, co, cls, f);
-      finish<D2Q9, COLL>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, false, f);
+      finish<D2Q9, COLL, MODE == kModeFirst>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, false, f);
       tile_store<DST, MODE>(c, dst, co, f);
       return;
     }
@@ -267,7 +267,7 @@ k_viv_fused(StepCtx c_arg, VsxIB2D ib, const typename SRC::T *__restrict__ src, 
   } else {
     local<D2Q9, SRC>(c, src, cell_of<D2Q9>(c, co[0], co[1], 0), f);
   }
-  finish<D2Q9, COLL>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, false, f);
+  finish<D2Q9, COLL, MODE == kModeFirst>(c, cell_of<D2Q9>(c, co[0], co[1], 0), co, org, false, f);
   tile_store<DST, MODE>(c, dst, co, f);
 }
 
