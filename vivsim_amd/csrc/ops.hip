@@ -214,12 +214,13 @@ __global__ void k_wall(VsxWall w, const float *__restrict__ fpre, const float *f
 }
 
 // The same on a copy of a small field in one launch: each thread takes a cell
-// through, the wall's with the wall update.  As a copy and a wall kernel the second
-// adds 4 us (512 x 400 cells: 4.2 + 4.4 us).  Large fields keep those two: the
-// library's copy moves 16 bytes a thread (129 x 97 x 110 cells: 31 + 15 us against 46
-// us; copying around the wall's cells by 16 bytes took 62 us, its index
-// arithmetic bounds it).
-constexpr size_t kWallCopyBytes = size_t(32) << 20;
+// through, the wall's with the wall update.  Up to 2 MB the calls are bound by
+// their launches, and one is saved (us per call, copy and wall kernel -> this one:
+// 128 x 128 13.7 -> 11.1, 24^3 13.9 -> 11.3 to 12.9).  Above it the library's copy,
+// which moves 16 bytes a thread, and the wall kernel are faster, the more so for
+// the walls of the last axis (32^3, 2.4 MB: 14.1 and 12.8 to 15.2; 40^3, 4.6 MB: 14.1
+// and 18.7 to 20.6; 512 x 400, 7 MB: 13.5 and 18).
+constexpr size_t kWallCopyBytes = size_t(2) << 20;
 
 template <class L>
 __global__ __launch_bounds__(kBlock) void k_wall_copy(VsxWall w, const float *__restrict__ fpre,
