@@ -244,6 +244,34 @@ def test_sphere_16bit_matches_oracle(sim, storage, tol):
     assert_close(got, f, tol, f"sphere f ({storage})")
 
 
+@pytest.mark.parametrize("variant,pipelined", [
+    (dict(cx=7.0, n_iter=3), False), (dict(cx=33.0, n_iter=1, collision="mrt"), False), (dict(cx=7.0, n_iter=0), False),
+    (dict(n_markers=2100, n_iter=3), False), (dict(n_markers=2100, n_iter=1, forcing="guo"), True),
+    (dict(n_markers=257), True)],
+    ids=["inlet_3it", "outlet_1it", "inlet_no_ib", "lists_over_64", "lists_over_64_pipelined", "odd_pipelined"])
+def test_sphere_window_and_marker_limits(sim, variant, pipelined):
+    """The window on a walled face (its cells go through the wall update), cells
+    with more stencil slots than a wavefront has lanes, marker counts that are no
+    multiple of a workgroup.  Tolerances as in test_sphere_matches_oracle."""
+    oc, pc = small_sphere(S.Sphere3D, **variant), small_sphere(sim.SphereCase, **variant)
+    steps = 6
+    say(f"sphere limits {variant} pipelined={pipelined}")
+    solver = sim.Sphere3D(pc, pipelined=pipelined)
+    if variant.get("n_markers") == 2100:
+        ptr = to_np(solver.cell_ptr)
+        assert np.diff(ptr).max() > 64
+    f0 = oc.initial_f(np.float64)
+    got, hh = solver.run(dev(f0), steps)
+    W, I = oc.stencil(np.float32)
+    f, hs = f0.astype(np.float64), []
+    for _ in range(steps):
+        f, h = S.sphere_step(oc, f, W.astype(np.float64), I)
+        hs.append(h)
+    assert_close(got, f, 5e-5, "sphere f")
+    if oc.n_iter > 0:
+        assert_close(hh, np.array(hs), 1e-4, "sphere force history")
+
+
 def test_sphere_transpose_is_exact(sim):
     """The transposed stencil lists every in-range slot once, per cell in ascending order."""
     pc = small_sphere(sim.SphereCase)
