@@ -532,12 +532,14 @@ __device__ __forceinline__ void edge_cells(const StepCtx &c, const EdgeList &E, 
 // (and z in 3D) the others, so a wavefront touches 64 consecutive cells.
 // k_bulk_walls: walls on several axes; the
 // first `edge_rows` rows of the outermost grid axis hold the cells on several
-// walls.  Their long chains (a few waves) run beside the bulk, and the
-// kernel keeps the register budget of the bulk path (waves_per_eu): what the
-// edge path needs above it is spilled there.
+// walls.  Their long chains (a few waves) run beside the bulk.  waves_per_eu sets
+// the registers of both paths: in 2D those of the bulk path, what the edge path needs
+// above it is spilled there; in 3D the bulk path with its walls spills too below
+// 128 registers (MRT cavity, us per operation at 5, 4, 3 waves: 32^3 18.3, 13.6,
+// 12.5; 96^3 36.0, 35.4, 39.4; 121 x 113 x 127 84.7, 68.6, 66.4).
 template <class L>
 constexpr int bulk_waves() {
-  return L::D == 2 ? 8 : 5;
+  return L::D == 2 ? 8 : 4;
 }
 
 template <class L, int COLL, int PHASE, class SRC, class DST>
