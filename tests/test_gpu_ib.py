@@ -140,29 +140,3 @@ def test_dyn(V):
     tq = V.dyn.get_torque_to_obj(dev(x0), dev(y0), 5.0, 6.0, np.zeros(3), dev(hm))
     assert math.isclose(float(tq), OD.get_torque_to_obj(x0.astype(np.float64), y0.astype(np.float64), 5.0, 6.0,
                                                         np.zeros(3), hm.astype(np.float64)), rel_tol=1e-6)
-
-
-@pytest.mark.parametrize("m,c,side,n_iter", [(1, 2, 6, 3), (120, 2, 50, 3), (511, 2, 110, 2), (513, 2, 111, 2), (1024, 2, 110, 1),
-                                             (1025, 2, 110, 1), (2048, 2, 90, 1), (2049, 2, 90, 1), (341, 3, 20, 2), (342, 3, 21, 2)])
-def test_mdf_one_workgroup_limits(m, c, side, n_iter):
-    """Multi-direct forcing on both sides of the one-workgroup form's limits (24576 grid values: 2 x 110^2 and
-    3 x 20^3 are inside, 2 x 111^2 and 3 x 21^3 outside; 4096 marker components; 65536 marker points x components),
-    against the float64 oracle, with some stencils leaving the grid.  Tolerance: float32 sums of up to some
-    ten terms per iteration, 4e-6 of the largest value."""
-    from oracle import ib as OI
-    from vivsim_amd import ib
-    r = np.random.default_rng(m + side)
-    if c == 2:
-        pos = r.uniform(-1.0, side + 1.0, size=(m, 2)).astype(np.float32)
-        W, I = OI.get_ib_stencil(pos[:, 0], pos[:, 1], side, OI.KERNELS["peskin_4pt"], 2)
-    else:
-        pos = r.uniform(0.0, side - 1.0, size=(m, 3)).astype(np.float32)
-        W, I = OI.get_ib_stencil3d(pos, (side,) * 3, OI.KERNELS["peskin_4pt"], 2)
-    u = r.standard_normal((c,) + (side,) * c).astype(np.float32)
-    U = r.standard_normal((m, c)).astype(np.float32)
-    ds = r.uniform(0.02, 0.05, size=m).astype(np.float32)
-    g, h = ib.multi_direct_forcing(dev(u), dev(W), torch.as_tensor(I, device="cuda"), dev(U), dev(ds), n_iter)
-    g64, h64 = OI.multi_direct_forcing(u.astype(np.float64), W.astype(np.float64), I, U.astype(np.float64),
-                                       ds.astype(np.float64), n_iter)
-    assert_close(g, g64, 4e-6, "grid force")
-    assert_close(h, h64, 4e-6, "marker force")

@@ -109,92 +109,6 @@ __global__ void k_mdf_update(const float *__restrict__ ub, const float *__restri
   }
 }
 
-// The whole loop (ib/mdf.py:35-64) by one workgroup, the force grid in LDS: one
-// launch instead of 5 + 4 n_iter, each of which a small body leaves idle for most of
-// its 3-7 us (four steps of a 512 x 400 VIV from the pure functions, 120 markers,
-// 3 iterations: 1.45 -> 1.27 ms).  Item t = marker x
-// component lives on thread t % 1024; the sums run over the stencil points in the
-// order of k_interp.
-constexpr int kMdfThreads = 1024, kMdfItems = 4;
-constexpr int64_t kMdfGrid = 24576;    // grid values in LDS (96 KiB)
-constexpr int64_t kMdfSlots = 65536;   // marker x point x component: more is faster spread over the CUs
-
-__global__ __launch_bounds__(kMdfThreads) void k_mdf_one(const float *__restrict__ grid_u, int c, int ng,
-                                                         const float *__restrict__ W, const int32_t *__restrict__ I,
-                                                         int m, int s, const float *__restrict__ U,
-                                                         const float *__restrict__ ds_arr, float ds, int n_iter,
-                                                         float *__restrict__ grid_force,
-                                                         float *__restrict__ marker_force) {
-  extern __shared__ float lds[];
-  float *grid = lds, *val = lds + c * ng;   // val[m][c]: what is being spread
-  const int tid = threadIdx.x, mc = m * c;
-  float ub[kMdfItems], F[kMdfItems];
-  auto interp = [&](const float *g, float scale, int t) {
-    const int k = t / c, comp = t % c;
-    float acc = 0.f;
-    for (int q = 0; q < s; ++q) acc += W[k * s + q] * (g[comp * ng + gather_index32(I[k * s + q], ng)] * scale);
-    return acc;
-  };
-  auto spread = [&]() {   // ends with a barrier
-    for (int i = tid; i < c * ng; i += kMdfThreads) grid[i] = 0.f;
-    __syncthreads();
-    // a wave per component takes the points in order: the sums do not depend on
-    // which wave comes first
-    const int comp = tid >> 6, ms = m * s;
-    if (comp < c) {
-      for (int t0 = tid & 63; t0 < ms; t0 += 256) {
-        int g[4];
-        float v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int t = t0 + 64 * u;
-          g[u] = t < ms ? scatter_index32(I[t], ng) : -1;
-          v[u] = g[u] >= 0 ? val[t / s * c + comp] * W[t] : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (g[u] >= 0) unsafeAtomicAdd(&grid[comp * ng + g[u]], v[u]);
-      }
-    }
-    __syncthreads();
-  };
-#pragma unroll
-  for (int j = 0; j < kMdfItems; ++j) {
-    const int t = tid + j * kMdfThreads;
-    F[j] = 0.f;
-    ub[j] = t < mc ? interp(grid_u, 1.0f, t) : 0.f;
-  }
-  for (int it = 0; it < n_iter; ++it) {
-#pragma unroll
-    for (int j = 0; j < kMdfItems; ++j) {
-      const int t = tid + j * kMdfThreads;
-      if (t < mc) {
-        const float d2 = (ds_arr ? ds_arr[t / c] : ds) * 2.0f;
-        const float v = (U[t] - ub[j]) * d2;
-        val[t] = v;
-        F[j] += v;
-      }
-    }
-    spread();
-#pragma unroll
-    for (int j = 0; j < kMdfItems; ++j) {
-      const int t = tid + j * kMdfThreads;
-      if (t < mc) ub[j] += interp(grid, 0.5f, t);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int j = 0; j < kMdfItems; ++j) {
-    const int t = tid + j * kMdfThreads;
-    if (t < mc) {
-      val[t] = F[j];
-      marker_force[t] = -F[j];
-    }
-  }
-  spread();
-  for (int i = tid; i < c * ng; i += kMdfThreads) grid_force[i] = grid[i];
-}
-
 __global__ void k_neg(const float *__restrict__ a, float *__restrict__ out, int64_t n) {
   GS_LOOP(i, n) out[i] = -a[i];
 }
@@ -460,12 +374,6 @@ static int mdf_run(const float *grid_u, int32_t c, int64_t ng, const float *W, c
                    const float *U, const float *ds_arr, float ds, int32_t n_iter, float *grid_force,
                    float *marker_force, float *work, void *stream) {
   const int64_t mc = (int64_t)m * c, ms = (int64_t)m * s;
-  if (c <= kMdfThreads / 64 && c * ng <= kMdfGrid && mc <= kMdfThreads * kMdfItems && ms * c <= kMdfSlots) {
-    hipLaunchKernelGGL(k_mdf_one, dim3(1), dim3(kMdfThreads), sizeof(float) * (size_t)(c * ng + mc), as_stream(stream),
-                       grid_u, c, (int)ng, W, I, m, s, U, ds_arr, ds, n_iter, grid_force, marker_force);
-    VSX_CHECK_LAUNCH();
-    return VSX_OK;
-  }
   float *ub = work, *F = work + mc, *dF = work + 2 * mc;
   L1(k_fill, (int64_t)c * ng, grid_force, 0.f, (int64_t)c * ng);
   L1(k_fill, mc, F, 0.f, mc);
