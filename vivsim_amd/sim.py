@@ -448,7 +448,7 @@ class Sphere3D:
     runs on a second stream while the bulk pass of step t streams.  The
     default is the sequential form: the sphere's IB kernels are multi-
     workgroup kernels that, run beside the bulk pass, get too few compute
-    units and make the pipelined step slower (0.24 against 0.16 ms at
+    units and make the pipelined step slower (0.24 against 0.15 ms at
     256 x 128 x 128)."""
 
     def __init__(self, case: SphereCase, storage="f32", pipelined=False):
