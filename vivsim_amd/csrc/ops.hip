@@ -207,8 +207,21 @@ __global__ void k_wall(VsxWall w, const float *__restrict__ fpre, const float *f
     float v[L::Q];
     const int64_t cw = wall_cell<L>(w.loc, j, 0, d);
     load_q<L>(f, n, cw, v);
-    apply_wall<L>(w, j, v, [&](float (&fn)[L::Q]) { load_q<L>(f, n, wall_cell<L>(w.loc, j, 1, d), fn); },
-                  [&](float (&fp)[L::Q]) { load_q<L>(fpre, n, cw, fp); });
+    // all sets are asked for at once: a wall's few waves wait for memory only
+    float fn[L::Q], fp[L::Q];
+    if (wall_needs_neighbor(w)) {
+      load_q<L>(f, n, wall_cell<L>(w.loc, j, 1, d), fn);
+    } else {
+#pragma unroll
+      for (int i = 0; i < L::Q; ++i) fn[i] = 0.f;
+    }
+    if (wall_needs_pre(w)) {
+      load_q<L>(fpre, n, cw, fp);
+    } else {
+#pragma unroll
+      for (int i = 0; i < L::Q; ++i) fp[i] = 0.f;
+    }
+    apply_wall<L>(w, j, v, Held<L::Q>{fn}, Held<L::Q>{fp});
     store_q<L>(out, n, cw, v);
   }
 }
