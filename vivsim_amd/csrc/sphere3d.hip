@@ -570,7 +570,7 @@ int sphere_run(const VsxLbm *p, const VsxIB3D *ib, const float *f_in, float *f_o
   VSX_REQUIRE(n <= 1 || wb, "need two work buffers for more than one step");
   hipStream_t s = as_stream(stream);
   const IB3DDev d = make_dev(*ib);
-  const StepCtx c = make_ctx<D3Q19>(*p, Window{d.origin, d.g_win, {ib->win[0], ib->win[1], ib->win[2]}});
+  const StepCtx3 c = make_ctx<D3Q19>(*p, Window{d.origin, d.g_win, {ib->win[0], ib->win[1], ib->win[2]}});
   if (n == 0) {
     if (f_out != f_in) VSX_HIP(hipMemcpyAsync(f_out, f_in, sizeof(float) * 19 * c.n, hipMemcpyDeviceToDevice, s));
     return VSX_OK;
@@ -610,15 +610,15 @@ int sphere_run(const VsxLbm *p, const VsxIB3D *ib, const float *f_in, float *f_o
     VSX_HIP(hipEventRecord(r->join_b, r->b));
     VSX_HIP(hipStreamWaitEvent(s, r->join_s, 0));
     VSX_HIP(hipStreamWaitEvent(s, r->join_b, 0));
-    const StepCtx cs = make_ctx<D3Q19>(*p, Window{nullptr, nullptr, {0, 0, 0}});
+    const StepCtx3 cs = make_ctx<D3Q19>(*p, Window{nullptr, nullptr, {0, 0, 0}});
     return step_any<D3Q19>(cs, cur, false, f_out, true, VSX_PHASE_STREAM, s);
   }
   // the window's cells gather their force from the markers' in the bulk pass
-  StepCtx cb = c;
-  cb.win.F = d.F;
-  cb.win.W = d.W;
-  cb.win.cell_ptr = d.cell_ptr;
-  cb.win.cell_slot = d.cell_slot;
+  StepCtx3 cb = c;
+  cb.F = d.F;
+  cb.W = d.W;
+  cb.cell_ptr = d.cell_ptr;
+  cb.cell_slot = d.cell_slot;
   for (int t = 0; t < n; ++t) {
     void *dst = bufs[t & 1];
     rc = ib3d_phase(c, d, cur, t == 0, ib->hist_h && t > 0 ? ib->hist_h + 3 * (int64_t)(t - 1) : nullptr, s);
@@ -628,7 +628,7 @@ int sphere_run(const VsxLbm *p, const VsxIB3D *ib, const float *f_in, float *f_o
     cur = dst;
   }
   if (ib->hist_h) hipLaunchKernelGGL(k_hist3d, dim3(1), dim3(256), 0, s, d, ib->hist_h + 3 * (int64_t)(n - 1));
-  const StepCtx cs = make_ctx<D3Q19>(*p, Window{nullptr, nullptr, {0, 0, 0}});
+  const StepCtx3 cs = make_ctx<D3Q19>(*p, Window{nullptr, nullptr, {0, 0, 0}});
   return step_any<D3Q19>(cs, cur, false, f_out, true, VSX_PHASE_STREAM, s);
 }
 

@@ -37,11 +37,6 @@ struct Window {
   const int32_t *origin;   // [3] clamped window origin, or null (no window)
   const float *g;          // [D][S0][S1(][S2)]
   int32_t size[3];
-  // 3D: the forces `F` [M][3] of the markers, gathered by the window's cells
-  // themselves (null: read from g); stencil weights and cell -> slot lists of
-  // vsx_ib3d_transpose_stencil, `points` slots per marker; also stored in g
-  const float *F = nullptr, *W = nullptr;
-  const int32_t *cell_ptr = nullptr, *cell_slot = nullptr;
 };
 
 // Sum over the stencil slots that land on window cell k of mf[m][a] * W[slot]
@@ -74,7 +69,9 @@ __device__ __forceinline__ void gather_cell3(const float *__restrict__ mf, const
   }
 }
 
-struct StepCtx {
+// Whole lines of the argument segment: every wave waits for the lines that hold
+// the grid's size and the pointers behind it before its first load.
+struct alignas(64) StepCtx {
   VsxLbm p;
   Window win;
   int32_t dims[3];         // nx, ny, nz (nz = 1 in 2D)
@@ -87,13 +84,27 @@ struct StepCtx {
   float shift[19];         // 16-bit storage: stored value = f_i - shift[i] = f_i - feq_i(1, p.store_u)
 };
 
+// 3D steps: the forces `F` [M][3] of the markers, gathered by the window's cells
+// themselves (null: read from win.g); stencil weights and cell -> slot lists of
+// vsx_ib3d_transpose_stencil; also stored in win.g.  Behind the rest, and in 3D only:
+// within Window these 32 bytes moved the grid's size across a line (periodic 3D runs, us
+// per step, within Window -> here: 32^3 4.47 -> 3.92, 64^3 9.01 -> 8.81, 65 x 64 x 63
+// 11.55 -> 11.37, 96^3 24.4 -> 24.2).
+struct StepCtx3 : StepCtx {
+  const float *F = nullptr, *W = nullptr;
+  const int32_t *cell_ptr = nullptr, *cell_slot = nullptr;
+};
+template <class L>
+using CtxOf = std::conditional_t<L::D == 3, StepCtx3, StepCtx>;
+
 // The kernel's StepCtx argument, addressed in the kernarg segment (it is always
 // the first kernel parameter, at offset 0).  Taking the context by reference
 // from here, instead of from the by-value parameter, keeps the compiler from
 // making a private per-lane copy of the ~1.4 KB block whenever a reference to
 // it reaches a function that is not inlined.
-__device__ __forceinline__ const StepCtx &kernel_ctx() {
-  return *reinterpret_cast<const StepCtx *>((const char *)__builtin_amdgcn_kernarg_segment_ptr());
+template <class CTX = StepCtx>
+__device__ __forceinline__ const CTX &kernel_ctx() {
+  return *reinterpret_cast<const CTX *>((const char *)__builtin_amdgcn_kernarg_segment_ptr());
 }
 
 // Cell index (< 2^31 cells, checked on the host).  Populations are addressed as
@@ -289,7 +300,7 @@ inline bool walls_need_edge(const VsxLbm &p) {
 // body force at a cell: uniform + optional full field + immersed-boundary window
 // (window origin `org`, used when `win`)
 template <class L>
-__device__ __forceinline__ void body_force(const StepCtx &c, uint32_t cell, const int (&co)[3], const int (&org)[3],
+__device__ __forceinline__ void body_force(const CtxOf<L> &c, uint32_t cell, const int (&co)[3], const int (&org)[3],
                                            bool win, float (&g)[3]) {
 #pragma unroll
   for (int a = 0; a < 3; ++a) g[a] = a < L::D ? c.p.g_uniform[a] : 0.f;
@@ -311,9 +322,9 @@ __device__ __forceinline__ void body_force(const StepCtx &c, uint32_t cell, cons
       for (int a = 1; a < L::D; ++a) k = k * c.win.size[a] + r[a];
       const int wn = c.win.size[0] * c.win.size[1] * (L::D == 3 ? c.win.size[2] : 1);
       if constexpr (L::D == 3) {
-        if (c.win.F) {
+        if (c.F) {
           float s[3];
-          gather_cell3(c.win.F, c.win.W, c.win.cell_ptr, c.win.cell_slot, k, s);
+          gather_cell3(c.F, c.W, c.cell_ptr, c.cell_slot, k, s);
 #pragma unroll
           for (int a = 0; a < 3; ++a) {
             const_cast<float *>(c.win.g)[a * wn + k] = s[a];
@@ -428,7 +439,7 @@ __device__ __forceinline__ void finish_unforced(const StepCtx &c, float (&f)[L::
 }
 
 template <class L, int COLL, bool IN_PLACE = false>
-__device__ __forceinline__ void finish(const StepCtx &c, uint32_t cell, const int (&co)[3], const int (&org)[3],
+__device__ __forceinline__ void finish(const CtxOf<L> &c, uint32_t cell, const int (&co)[3], const int (&org)[3],
                                        bool win, float (&f)[L::Q]) {
   bool unforced = !win && !c.p.g;
 #pragma unroll
@@ -463,7 +474,7 @@ struct EdgeList {
 // (scratch arrays, one chain of loads per level) these cells took 17 us of a
 // 256^2 cavity step and 120 us of a 121 x 113 x 127 one, as a kernel of their own.
 template <class L, int COLL, int PHASE, class SRC, class DST>
-__device__ __forceinline__ void edge_cells(const StepCtx &c, const EdgeList &E, int64_t t,
+__device__ __forceinline__ void edge_cells(const CtxOf<L> &c, const EdgeList &E, int64_t t,
                                            const typename SRC::T *__restrict__ src,
                                            typename DST::T *__restrict__ dst) {
   constexpr int G = 1 << L::D;
@@ -543,7 +554,7 @@ constexpr int bulk_waves() {
 }
 
 template <class L, int COLL, int PHASE, class SRC, class DST>
-__device__ __forceinline__ void bulk_cells(const StepCtx &c, int outer, const typename SRC::T *__restrict__ src,
+__device__ __forceinline__ void bulk_cells(const CtxOf<L> &c, int outer, const typename SRC::T *__restrict__ src,
                                            typename DST::T *__restrict__ dst) {
   int co[3];
   if constexpr (L::D == 2) {
@@ -580,17 +591,17 @@ __device__ __forceinline__ void bulk_cells(const StepCtx &c, int outer, const ty
 }
 
 template <class L, int COLL, int PHASE, class SRC, class DST>
-__global__ __launch_bounds__(256) void k_bulk(StepCtx c_arg, const typename SRC::T *__restrict__ src,
+__global__ __launch_bounds__(256) void k_bulk(CtxOf<L> c_arg, const typename SRC::T *__restrict__ src,
                                               typename DST::T *__restrict__ dst) {
-  bulk_cells<L, COLL, PHASE, SRC, DST>(kernel_ctx(), L::D == 2 ? blockIdx.y : blockIdx.z, src, dst);
+  bulk_cells<L, COLL, PHASE, SRC, DST>(kernel_ctx<CtxOf<L>>(), L::D == 2 ? blockIdx.y : blockIdx.z, src, dst);
 }
 
 template <class L, int COLL, int PHASE, class SRC, class DST>
 __global__ __attribute__((amdgpu_flat_work_group_size(64, 256),
                           amdgpu_waves_per_eu(bulk_waves<L>(), bulk_waves<L>()))) void
-k_bulk_walls(StepCtx c_arg, const typename SRC::T *__restrict__ src, typename DST::T *__restrict__ dst, EdgeList E,
+k_bulk_walls(CtxOf<L> c_arg, const typename SRC::T *__restrict__ src, typename DST::T *__restrict__ dst, EdgeList E,
             int edge_rows) {
-  const StepCtx &c = kernel_ctx();
+  const auto &c = kernel_ctx<CtxOf<L>>();
   const int outer = L::D == 2 ? blockIdx.y : blockIdx.z;
   if (outer < edge_rows) {
     const int64_t row = L::D == 2 ? (int64_t)outer : (int64_t)outer * gridDim.y + blockIdx.y;

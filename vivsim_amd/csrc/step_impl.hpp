@@ -25,8 +25,8 @@ int validate_lbm(const VsxLbm *p) {
 }
 
 template <class L>
-StepCtx make_ctx(const VsxLbm &p, Window win) {
-  StepCtx c;
+CtxOf<L> make_ctx(const VsxLbm &p, Window win) {
+  CtxOf<L> c;
   c.p = p;
   c.win = win;
   c.dims[0] = p.nx;
@@ -90,7 +90,7 @@ EdgeList make_edges(const StepCtx &c) {
 }
 
 template <class L, int COLL, int PHASE, class SRC, class DST>
-void launch_bulk(const StepCtx &c, const typename SRC::T *src, typename DST::T *dst, dim3 grid, dim3 block,
+void launch_bulk(const CtxOf<L> &c, const typename SRC::T *src, typename DST::T *dst, dim3 grid, dim3 block,
                  hipStream_t s) {
   if constexpr (PHASE != VSX_PHASE_COLLIDE) {
     if (c.p.n_walls > 0 && walls_need_edge<L>(c.p)) {
@@ -107,7 +107,7 @@ void launch_bulk(const StepCtx &c, const typename SRC::T *src, typename DST::T *
 }
 
 template <class L, int PHASE, class SRC, class DST>
-int launch_phase(const StepCtx &c, const void *src, void *dst, hipStream_t s) {
+int launch_phase(const CtxOf<L> &c, const void *src, void *dst, hipStream_t s) {
   dim3 grid, block;
   bulk_grid<L>(c, grid, block);
   auto S = static_cast<const typename SRC::T *>(src);
@@ -130,7 +130,7 @@ int launch_phase(const StepCtx &c, const void *src, void *dst, hipStream_t s) {
 
 // runtime (phase, src storage, dst storage) -> template instantiation
 template <class L, class ST>
-int phase_dispatch(const StepCtx &c, const void *src, bool src_f32, void *dst, bool dst_f32, int phase, hipStream_t s) {
+int phase_dispatch(const CtxOf<L> &c, const void *src, bool src_f32, void *dst, bool dst_f32, int phase, hipStream_t s) {
   using F32 = Store<VSX_STORE_F32>;
   switch (phase) {
     case VSX_PHASE_COLLIDE:
@@ -156,7 +156,7 @@ int phase_dispatch(const StepCtx &c, const void *src, bool src_f32, void *dst, b
 }
 
 template <class L>
-int step_any(const StepCtx &c, const void *src, bool src_f32, void *dst, bool dst_f32, int phase, hipStream_t s) {
+int step_any(const CtxOf<L> &c, const void *src, bool src_f32, void *dst, bool dst_f32, int phase, hipStream_t s) {
   switch (c.p.storage) {
     case VSX_STORE_F32: return phase_dispatch<L, Store<VSX_STORE_F32>>(c, src, true, dst, true, phase, s);
     case VSX_STORE_F16S: return phase_dispatch<L, Store<VSX_STORE_F16S>>(c, src, src_f32, dst, dst_f32, phase, s);
@@ -170,7 +170,7 @@ int step_entry(const VsxLbm *p, const void *src, int src_f32, void *dst, int dst
   int rc = validate_lbm<L>(p);
   if (rc) return rc;
   VSX_REQUIRE(src && dst && src != dst, "step needs distinct source and destination buffers");
-  const StepCtx c = make_ctx<L>(*p, Window{nullptr, nullptr, {0, 0, 0}});
+  const CtxOf<L> c = make_ctx<L>(*p, Window{nullptr, nullptr, {0, 0, 0}});
   return step_any<L>(c, src, src_f32 != 0, dst, dst_f32 != 0, phase, as_stream(stream));
 }
 
@@ -208,7 +208,7 @@ int run_entry(const VsxLbm *p, const float *f_in, float *f_out, void *wa, void *
   VSX_REQUIRE(n >= 0, "negative step count");
   VSX_REQUIRE(n <= 1 || wb, "need two work buffers for more than one step");
   hipStream_t s = as_stream(stream);
-  const StepCtx c = make_ctx<L>(*p, Window{nullptr, nullptr, {0, 0, 0}});
+  const CtxOf<L> c = make_ctx<L>(*p, Window{nullptr, nullptr, {0, 0, 0}});
   if (n == 0) {
     if (f_out != f_in) VSX_HIP(hipMemcpyAsync(f_out, f_in, sizeof(float) * L::Q * c.n, hipMemcpyDeviceToDevice, s));
     return VSX_OK;
