@@ -27,20 +27,18 @@
 
 namespace vsx {
 
-constexpr int kMaxOps = 8;   // operations per launch
-
 struct MultiArgs {
-  int32_t k;                  // operations of this launch (2 .. KL)
+  int32_t k;                  // operations of this launch (2 .. kRunOps)
   int32_t first, last;        // operation 1 is C / operation k is S
   int32_t nty, tiles;         // tiles along y, all tiles
   int32_t store;              // field stores: 0 plain, 1 non-temporal, 2 written through
-  uint32_t magic[kMaxOps];    // magic[e] = ceil(2^20 / (TY + 2 e)): division by the row length of a region
+  uint32_t magic[kRunOps];    // magic[e] = ceil(2^20 / (TY + 2 e)): division by the row length of a region
 };
 
-// TX x TY tile, at most KL operations, NT threads; a region of RX x RW cells in LDS
-template <int TX_, int TY_, int KL_, int NT_>
+// TX x TY tile, NT threads; a region of RX x RW cells in LDS
+template <int TX_, int TY_, int NT_>
 struct MultiCfg {
-  static constexpr int TX = TX_, TY = TY_, KL = KL_, NT = NT_;
+  static constexpr int TX = TX_, TY = TY_, KL = kRunOps, NT = NT_;
   static constexpr int RX = TX + 2 * (KL - 1), RW = TY + 2 * (KL - 1), RC = RX * RW;
   // waves per SIMD: two workgroups of 768 threads per CU, one of 1024 (whose wall
   // units then keep their three sets of populations in registers)
@@ -48,7 +46,7 @@ struct MultiCfg {
   // distance of the seam from its tile's edge: the wall cells on both sides of it,
   // their inward neighbours and those neighbours' own lie KL cells and more inside
   static constexpr int SX = KL + 2 > 8 ? 16 : 8, SY = TY >= 64 ? 16 : SX;
-  static_assert(KL <= kMaxOps && KL + 2 <= SX && SX + 3 <= TX && SY + 3 <= TY, "wall cells lie inside their tile");
+  static_assert(KL + 2 <= SX && SX + 3 <= TX && SY + 3 <= TY, "wall cells lie inside their tile");
   static_assert(NT % 64 == 0 && NT / 64 >= (RX > 64 || RW > 64 ? 12 : 8), "a wave for every wall and corner unit");
 };
 
@@ -271,7 +269,7 @@ int run_multi(const StepCtx &c, const float *f_in, float *f_out, void *wa, void 
   a.tiles = a.nty * ((c.dims[0] + CF::TX - 1) / CF::TX);
   const size_t bytes = sizeof(typename ST::T);
   a.store = (size_t)c.n * 9 * bytes > kLastLevelCacheBytes ? 1 : write_through(c.n, 9, c.dims[1], bytes) ? 2 : 0;
-  for (int e = 0; e < kMaxOps; ++e) a.magic[e] = ((1u << 20) + CF::TY + 2 * e - 1) / (CF::TY + 2 * e);
+  for (int e = 0; e < kRunOps; ++e) a.magic[e] = ((1u << 20) + CF::TY + 2 * e - 1) / (CF::TY + 2 * e);
   // n + 1 operations in launches of equal size (2 and more each)
   const int ops = n + 1, launches = (ops + CF::KL - 1) / CF::KL;
   const void *cur = f_in;
@@ -305,12 +303,12 @@ int run_multi_tiles(const StepCtx &c, const float *f_in, float *f_out, void *wa,
   auto tiles = [&](int tx, int ty) {
     return (int64_t)((c.dims[0] + tx - 1) / tx) * ((c.dims[1] + ty - 1) / ty);
   };
-  if (tiles(16, 16) <= 256) return run_multi<COLL, ST, MultiCfg<16, 16, 6, 1024>>(c, f_in, f_out, wa, wb, n, s);
-  if (tiles(16, 32) <= 512) return run_multi<COLL, ST, MultiCfg<16, 32, 6, 1024>>(c, f_in, f_out, wa, wb, n, s);
+  if (tiles(16, 16) <= 256) return run_multi<COLL, ST, MultiCfg<16, 16, 1024>>(c, f_in, f_out, wa, wb, n, s);
+  if (tiles(16, 32) <= 512) return run_multi<COLL, ST, MultiCfg<16, 32, 1024>>(c, f_in, f_out, wa, wb, n, s);
   if constexpr (sizeof(typename ST::T) == 2) {
-    if (tiles(40, 64) >= 512) return run_multi<COLL, ST, MultiCfg<40, 64, 6, 768>>(c, f_in, f_out, wa, wb, n, s);
+    if (tiles(40, 64) >= 512) return run_multi<COLL, ST, MultiCfg<40, 64, 768>>(c, f_in, f_out, wa, wb, n, s);
   }
-  return run_multi<COLL, ST, MultiCfg<20, 64, 6, 768>>(c, f_in, f_out, wa, wb, n, s);
+  return run_multi<COLL, ST, MultiCfg<20, 64, 768>>(c, f_in, f_out, wa, wb, n, s);
 }
 
 // One instantiation per storage, each in a translation unit of its own.

@@ -174,7 +174,8 @@ int step_entry(const VsxLbm *p, const void *src, int src_f32, void *dst, int dst
   return step_any<L>(c, src, src_f32 != 0, dst, dst_f32 != 0, phase, as_stream(stream));
 }
 
-// The multi-operation runs (multi2d.hpp), per storage.
+// The multi-operation runs (multi2d.hpp), per storage; operations per launch.
+constexpr int kRunOps = 6;
 int multi2d_run_f32(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
 int multi2d_run_f16(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
 int multi2d_run_bf16(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
@@ -182,12 +183,12 @@ int multi2d_run_e3m12(const StepCtx &, const float *, float *, void *, void *, i
 
 // Whether a run goes through them: sides that hold the seam and its rings inside
 // a tile, at most one wall per face, and an input that the output of a run of one
-// launch (up to 5 steps) does not overlap.
+// launch (n + 1 operations) does not overlap.
 inline bool multi2d_takes(const StepCtx &c, const float *f_in, const float *f_out, int n) {
   for (int l = 0; l < 4; ++l)
     if (c.order[l] == -2) return false;
   const int64_t pops = 9 * c.n, gap = f_in < f_out ? f_out - f_in : f_in - f_out;
-  return c.dims[0] >= 40 && c.dims[1] >= 40 && (n > 5 || gap >= pops);
+  return c.dims[0] >= 40 && c.dims[1] >= 40 && (n + 1 > kRunOps || gap >= pops);
 }
 
 inline int multi2d_run(const StepCtx &c, const float *f_in, float *f_out, void *wa, void *wb, int n, hipStream_t s) {
