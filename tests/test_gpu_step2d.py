@@ -377,3 +377,36 @@ def test_run_equals_single_passes(sim, shape, n, storage):
         f = f0.clone()
         m.run(f, n, out=f)
         assert torch.equal(f, ref), name + " in place"
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16s"])
+@pytest.mark.parametrize("n", [3, 6, 7, 13])
+def test_run_with_a_work_buffer(sim, n, storage):
+    """A run whose input is work_a (FP32: collided in place) or whose output is
+    either work buffer that is idle at its end gives the same populations as a run
+    between buffers of its own."""
+    from vivsim_amd import _lib as L
+    import ctypes
+    nx, ny = 97, 66
+    f0 = dev(rand_state(nx, ny))
+    m = sim.LBM((nx, ny), 1.7, collision="mrt", walls=WALLSETS["channel"], storage=storage)
+    ref = m.run(f0, n)
+    say(f"run with a work buffer: {n} steps {storage}")
+
+    def call(f_in, f_out, wa, wb):
+        L.call("vsx_d2q9_run", ctypes.byref(m.p), L.ptr(f_in), L.ptr(f_out), L.ptr(wa), L.ptr(wb), n)
+        return f_out
+
+    new = lambda: torch.empty_like(f0)   # as large as any storage needs
+    if storage == "f32":
+        wa = f0.clone()
+        assert torch.equal(call(wa, new(), wa, new()), ref)
+        wa = f0.clone()
+        idle = n % 2   # the last of the n operations before the closing one writes work (n - 1) % 2
+        w = [wa, new()]
+        assert torch.equal(call(wa, w[idle], *w), ref)
+    w = [new(), new()]
+    assert torch.equal(call(f0, w[n % 2], *w), ref)
+    if n > 6:   # in place over several launches
+        f = f0.clone()
+        assert torch.equal(call(f, f, new(), new()), ref)

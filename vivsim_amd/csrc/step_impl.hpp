@@ -182,13 +182,22 @@ int multi2d_run_bf16(const StepCtx &, const float *, float *, void *, void *, in
 int multi2d_run_e3m12(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
 
 // Whether a run goes through them: sides that hold the seam and its rings inside
-// a tile, at most one wall per face, and an input that the output of a run of one
-// launch (n + 1 operations) does not overlap.
-inline bool multi2d_takes(const StepCtx &c, const float *f_in, const float *f_out, int n) {
+// a tile, at most one wall per face, and no launch (run_multi) that reads a buffer
+// it writes.  Single passes also take an input that is work_a (collided in place) and
+// an output that is the work buffer idle at the end.
+inline bool multi2d_takes(const StepCtx &c, const float *f_in, const float *f_out, const void *wa, const void *wb,
+                          int n) {
   for (int l = 0; l < 4; ++l)
     if (c.order[l] == -2) return false;
-  const int64_t pops = 9 * c.n, gap = f_in < f_out ? f_out - f_in : f_in - f_out;
-  return c.dims[0] >= 40 && c.dims[1] >= 40 && (n + 1 > kRunOps || gap >= pops);
+  if (c.dims[0] < 40 || c.dims[1] < 40) return false;
+  const size_t f = 9 * (size_t)c.n * sizeof(float), w = 9 * (size_t)c.n * store_bytes(c.p.storage);
+  auto apart = [](const void *a, size_t na, const void *b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x + na <= y || y + nb <= x;
+  };
+  const int launches = (n + kRunOps) / kRunOps;   // of n + 1 operations
+  if (launches == 1) return apart(f_in, f, f_out, f);
+  return apart(f_in, f, wa, w) && apart(f_out, f, launches % 2 ? wb : wa, w);
 }
 
 inline int multi2d_run(const StepCtx &c, const float *f_in, float *f_out, void *wa, void *wb, int n, hipStream_t s) {
@@ -215,7 +224,7 @@ int run_entry(const VsxLbm *p, const float *f_in, float *f_out, void *wa, void *
     return VSX_OK;
   }
   if constexpr (L::D == 2) {
-    if (multi2d_takes(c, f_in, f_out, n)) return multi2d_run(c, f_in, f_out, wa, wb, n, s);
+    if (multi2d_takes(c, f_in, f_out, wa, wb, n)) return multi2d_run(c, f_in, f_out, wa, wb, n, s);
   }
   rc = step_any<L>(c, f_in, true, wa, false, VSX_PHASE_COLLIDE, s);
   if (rc) return rc;
