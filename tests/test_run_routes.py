@@ -34,6 +34,9 @@ int main() {
   p.ny = 50;
   p.nz = 1;
   int bad = 0;
+  for (int n = INT_MAX - 8; n > 0 && n <= INT_MAX - 1; ++n) bad += run_launches(n) != n / kRunOps + 1;
+  bad += run_launches(INT_MAX) != INT_MAX / kRunOps + 1 || run_launches(5) != 1 || run_launches(6) != 2;
+  if (bad) printf("launches of the longest runs\n");
   for (int storage = 0; storage < 2; ++storage) {
     p.storage = storage;
     const StepCtx c = make_ctx<D2Q9>(p, Window{nullptr, nullptr, {0, 0, 0}});

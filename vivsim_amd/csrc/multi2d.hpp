@@ -271,11 +271,11 @@ int run_multi(const StepCtx &c, const float *f_in, float *f_out, void *wa, void 
   a.store = (size_t)c.n * 9 * bytes > kLastLevelCacheBytes ? 1 : write_through(c.n, 9, c.dims[1], bytes) ? 2 : 0;
   for (int e = 0; e < kRunOps; ++e) a.magic[e] = ((1u << 20) + CF::TY + 2 * e - 1) / (CF::TY + 2 * e);
   // n + 1 operations in launches of equal size (2 and more each)
-  const int ops = n + 1, launches = (ops + CF::KL - 1) / CF::KL;
+  const int64_t ops = (int64_t)n + 1, launches = run_launches(n);
   const void *cur = f_in;
   void *bufs[2] = {wa, wb};
-  for (int j = 0, done = 0; j < launches; ++j) {
-    a.k = (ops - done + launches - j - 1) / (launches - j);
+  for (int64_t j = 0, done = 0; j < launches; ++j) {
+    a.k = (int)((ops - done + launches - j - 1) / (launches - j));
     a.first = j == 0;
     a.last = j == launches - 1;
     void *dst = a.last ? f_out : bufs[j & 1];

@@ -176,6 +176,8 @@ int step_entry(const VsxLbm *p, const void *src, int src_f32, void *dst, int dst
 
 // The multi-operation runs (multi2d.hpp), per storage; operations per launch.
 constexpr int kRunOps = 6;
+// launches of a run of n steps, n + 1 operations (64 bits: n may be the largest int)
+inline int64_t run_launches(int n) { return ((int64_t)n + kRunOps) / kRunOps; }
 int multi2d_run_f32(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
 int multi2d_run_f16(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
 int multi2d_run_bf16(const StepCtx &, const float *, float *, void *, void *, int, hipStream_t);
@@ -195,7 +197,7 @@ inline bool multi2d_takes(const StepCtx &c, const float *f_in, const float *f_ou
     const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
     return x + na <= y || y + nb <= x;
   };
-  const int launches = (n + kRunOps) / kRunOps;   // of n + 1 operations
+  const int64_t launches = run_launches(n);
   if (launches == 1) return apart(f_in, f, f_out, f);
   return apart(f_in, f, wa, w) && apart(f_out, f, launches % 2 ? wb : wa, w);
 }
