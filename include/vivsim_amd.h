@@ -219,9 +219,10 @@ const char *vsx_version(void);
 const char *vsx_last_error(void);
 int vsx_device_sync(void);
 /* Instrumentation (no counterpart in the reference): between start and stop the
- * fused drivers record a HIP event pair, on their stream, around every
- * VSX_PHASE_FULL bulk kernel (at most max_pairs); stop synchronises on the last
- * pair and returns the per-launch durations in milliseconds. */
+ * fused drivers record a HIP event pair, on their stream, around every bulk
+ * kernel with VSX_PHASE_FULL steps (at most max_pairs steps); stop synchronises on
+ * the last pair and returns the duration of each such step in milliseconds: of
+ * its launch, or, where a launch takes k operations (2D runs), a k-th of it. */
 int vsx_timer_start(int32_t max_pairs);
 int vsx_timer_stop(float *ms, int32_t max, int32_t *n_out);
 

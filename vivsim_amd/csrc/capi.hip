@@ -34,7 +34,8 @@ int fail(int code, const char *fmt, ...) {
 namespace {
 struct Timer {
   std::vector<hipEvent_t> a, b;
-  int n = 0;
+  std::vector<int> ops, full;   // operations of the launch between a pair, full steps among them
+  int n = 0, steps = 0;         // pairs recorded, full steps in them
   bool on = false;
 };
 Timer g_timer;
@@ -47,12 +48,16 @@ static bool capturing(hipStream_t s) {
 }
 
 void timer_begin(hipStream_t s) {
-  if (g_timer.on && g_timer.n < (int)g_timer.a.size() && !capturing(s)) (void)hipEventRecord(g_timer.a[g_timer.n], s);
+  if (g_timer.on && g_timer.steps < (int)g_timer.a.size() && !capturing(s))
+    (void)hipEventRecord(g_timer.a[g_timer.n], s);
 }
 
-void timer_end(hipStream_t s) {
-  if (g_timer.on && g_timer.n < (int)g_timer.a.size() && !capturing(s)) {
+void timer_end(hipStream_t s, int ops, int full) {
+  if (g_timer.on && g_timer.steps < (int)g_timer.a.size() && !capturing(s)) {
     (void)hipEventRecord(g_timer.b[g_timer.n], s);
+    g_timer.ops[g_timer.n] = ops;
+    g_timer.full[g_timer.n] = full;
+    g_timer.steps += full;
     ++g_timer.n;
   }
 }
@@ -120,7 +125,9 @@ extern "C" int vsx_timer_start(int32_t max_pairs) {
     g_timer.a.push_back(x);
     g_timer.b.push_back(y);
   }
-  g_timer.n = 0;
+  g_timer.ops.resize(g_timer.a.size());
+  g_timer.full.resize(g_timer.a.size());
+  g_timer.n = g_timer.steps = 0;
   g_timer.on = true;
   return VSX_OK;
 }
@@ -128,10 +135,14 @@ extern "C" int vsx_timer_start(int32_t max_pairs) {
 extern "C" int vsx_timer_stop(float *ms, int32_t max, int32_t *n_out) {
   using vsx::g_timer;
   g_timer.on = false;
-  const int n = g_timer.n < max ? g_timer.n : max;
-  if (n > 0) VSX_HIP(hipEventSynchronize(g_timer.b[n - 1]));
-  for (int i = 0; i < n; ++i) VSX_HIP(hipEventElapsedTime(&ms[i], g_timer.a[i], g_timer.b[i]));
-  if (n_out) *n_out = n;
+  const int steps = g_timer.steps < max ? g_timer.steps : max;
+  if (steps > 0) VSX_HIP(hipEventSynchronize(g_timer.b[g_timer.n - 1]));
+  for (int i = 0, k = 0; k < steps; ++i) {
+    float t = 0.f;
+    VSX_HIP(hipEventElapsedTime(&t, g_timer.a[i], g_timer.b[i]));
+    for (int j = 0; j < g_timer.full[i] && k < steps; ++j) ms[k++] = t / (float)g_timer.ops[i];
+  }
+  if (n_out) *n_out = steps;
   return VSX_OK;
 }
 

@@ -12,9 +12,10 @@
 namespace vsx {
 
 void set_error(const char *fmt, ...);
-// event pair around a kernel launch while vsx_timer_start() is active
+// event pair around a kernel launch while vsx_timer_start() is active; the launch
+// holds `ops` operations, `full` (>= 1) of them full steps
 void timer_begin(hipStream_t s);
-void timer_end(hipStream_t s);
+void timer_end(hipStream_t s, int ops = 1, int full = 1);
 int fail(int code, const char *fmt, ...);
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
