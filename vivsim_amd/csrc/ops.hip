@@ -188,16 +188,18 @@ struct Dims {
   int n[3];
 };
 
-// cell index of wall node j at layer `layer` (0 = wall line, 1 = first inward neighbour)
+// cell index of wall node j at layer `layer` (0 = wall line, 1 = first inward neighbour).
+// Coordinates by selects: an array indexed by the axis goes to LDS, and a kernel with
+// such an array reads the size of its workgroup from the dispatch packet, in host memory,
+// in every wave (k_wall_copy at 229 x 253 16.0 us with the array, 3.6 without; k_wall
+// 1 us less).
 template <class L>
 __device__ __forceinline__ int64_t wall_cell(int loc, int64_t j, int layer, Dims d) {
-  const int a = L::w_axis[loc], sg = L::w_sign[loc];
-  const int idx = sg > 0 ? layer : d.n[a] - 1 - layer;
-  int co[3];
-  if (a == 0) { co[0] = idx; co[1] = (int)(j / d.n[2]); co[2] = (int)(j % d.n[2]); }
-  else if (a == 1) { co[1] = idx; co[0] = (int)(j / d.n[2]); co[2] = (int)(j % d.n[2]); }
-  else { co[2] = idx; co[0] = (int)(j / d.n[1]); co[1] = (int)(j % d.n[1]); }
-  return ((int64_t)co[0] * d.n[1] + co[1]) * d.n[2] + co[2];
+  const int a = L::w_axis[loc], sg = L::w_sign[loc], n0 = d.n[0], n1 = d.n[1], n2 = d.n[2];
+  const int idx = sg > 0 ? layer : (a == 0 ? n0 : (a == 1 ? n1 : n2)) - 1 - layer;
+  const int row = a == 2 ? n1 : n2, p = (int)(j / row), q = (int)(j % row);
+  const int x = a == 0 ? idx : p, y = a == 0 ? p : (a == 1 ? idx : q), z = a == 2 ? idx : q;
+  return ((int64_t)x * n1 + y) * n2 + z;
 }
 
 template <class L>
@@ -227,19 +229,20 @@ __global__ void k_wall(VsxWall w, const float *__restrict__ fpre, const float *f
 }
 
 // The same on a copy of a small field in one launch: each thread takes a cell
-// through, the wall's with the wall update.  Up to 2 MB the calls are bound by
-// their launches, and one is saved (us per call, copy and wall kernel -> this one:
-// 128 x 128 13.7 -> 11.1, 24^3 13.9 -> 11.3 to 12.9).  Above it the library's copy,
-// which moves 16 bytes a thread, and the wall kernel are faster, the more so for
-// the walls of the last axis (32^3, 2.4 MB: 14.1 and 12.8 to 15.2; 40^3, 4.6 MB: 14.1
-// and 18.7 to 20.6; 512 x 400, 7 MB: 13.5 and 18).
+// through, the wall's with the wall update.  The calls are bound by their launches,
+// and one is saved (us per call, copy and wall kernel -> this one: 128 x 128 12.8 -> 10.9,
+// 20^3 13.0 -> 11.3, 30^3, 2.05 MB, 13.0 -> 11.3; kernels alone 4.4 to 5.8 -> 3.2 to 4.5,
+// 5.6 to 9.2 -> 5.4 to 9.1, 5.9 to 11.2 -> 5.8 to 8.2).  The limit lies where the gain was first
+// measured, not where it ends (a copy of this code that takes all sizes: 40^3, 4.9 MB,
+// 13.0 -> 11.3; 512 x 400, 7.4 MB, 12.9 -> 11.1; 64^3, 20 MB, 12.8 to 23.3 -> 11.1 to 12.3).
 constexpr size_t kWallCopyBytes = size_t(2) << 20;
 
 template <class L>
 __global__ __launch_bounds__(kBlock) void k_wall_copy(VsxWall w, const float *__restrict__ fpre,
                                                       const float *__restrict__ f, float *__restrict__ out, Dims d) {
   const int64_t n = (int64_t)d.n[0] * d.n[1] * d.n[2];
-  const int a = L::w_axis[w.loc], face = L::w_sign[w.loc] > 0 ? 0 : d.n[a] - 1;
+  const int a = L::w_axis[w.loc];
+  const int face = L::w_sign[w.loc] > 0 ? 0 : (a == 0 ? d.n[0] : (a == 1 ? d.n[1] : d.n[2])) - 1;
   VSX_GRID_STRIDE(c, n) {
     int x, y, z;
     cell_coords(c, n, d.n[1], d.n[2], x, y, z);
