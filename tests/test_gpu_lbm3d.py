@@ -308,3 +308,22 @@ def test_cells_on_several_walls(sim, shape, walls):
     for _ in range(4):
         ref = S3.lbm_step3d(ref, 1.6, W, "bgk")
     assert_close(got, ref, 2e-5, f"{walls} {shape}")
+
+
+def test_sphere_window_of_several_spread_launches(sim):
+    """A window of more cells (130^3) than one launch of the spread takes (2^21).
+    Tolerances as in test_sphere_matches_oracle."""
+    kw = dict(nx=140, ny=134, nz=134, D=124.0, cx=67.0, cy=67.0, cz=67.0, n_markers=48000)
+    oc, pc = small_sphere(S.Sphere3D, **kw), small_sphere(sim.SphereCase, **kw)
+    assert pc.ib_size ** 3 > 1 << 21
+    say(f"sphere window {pc.ib_size}^3")
+    solver = sim.Sphere3D(pc)
+    f0 = oc.initial_f(np.float64)
+    got, hh = solver.run(dev(f0), 2)
+    W, I = oc.stencil(np.float32)
+    f, hs = f0.astype(np.float64), []
+    for _ in range(2):
+        f, h = S.sphere_step(oc, f, W.astype(np.float64), I)
+        hs.append(h)
+    assert_close(got, f, 5e-5, "sphere f")
+    assert_close(hh, np.array(hs), 1e-4, "sphere force history")

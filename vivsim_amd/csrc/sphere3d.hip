@@ -202,16 +202,19 @@ __global__ __launch_bounds__(256) void k_mark3d(IB3DDev d, int it) {
 // out[a][k] = sum over the stencil slots that land on window cell k of
 // mf[m][a] * W[slot] (ib/stencil.py:81-110 as a gather), in slot order.  Eight lanes
 // per cell: each loads every eighth slot of the list, eight in flight, and the
-// group then adds them up in order, lane after lane.  agent: into planes, else [cells][3].  (A thread per cell walks its
-// list of up to some 60 slots in dependent round trips: 9.4 us at 4096 markers,
-// 7.4 so.)
+// group then adds them up in order, lane after lane.  agent: into planes, else
+// [cells][3].  (A thread per cell walks its list of up to some 60 slots in dependent
+// round trips: 9.4 us at 4096 markers, 7.4 so.)  A launch takes kSpreadCells cells from
+// k0 on: eight lanes per cell of the largest windows are more threads than a launch
+// may have (2^32).
+constexpr int64_t kSpreadCells = (int64_t)1 << 21;
 template <int I>
 __device__ __forceinline__ float group8_get(float v) {   // lane I of each group of eight
   return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (I << 5) | 0x18));
 }
 __global__ __launch_bounds__(256) void k_spread3d(IB3DDev d, const float *__restrict__ mf, float *__restrict__ out,
-                                                  bool agent) {
-  const int64_t k = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 3;
+                                                  bool agent, int64_t k0) {
+  const int64_t k = k0 + ((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 3);
   const int i = threadIdx.x & 7;
   if (k - ((threadIdx.x & 63) >> 3) >= d.cells) return;   // whole wavefronts
   const bool on = k < d.cells;
@@ -481,6 +484,13 @@ void win_u_any(const StepCtx &c, const IB3DDev &d, const void *src, bool first, 
   }
 }
 
+void launch_spread(const IB3DDev &d, const float *mf, float *out, bool agent, hipStream_t s) {
+  for (int64_t k0 = 0; k0 < d.cells; k0 += kSpreadCells) {
+    const int64_t cells = d.cells - k0 < kSpreadCells ? d.cells - k0 : kSpreadCells;
+    hipLaunchKernelGGL(k_spread3d, dim3((unsigned)((8 * cells + 255) / 256)), dim3(256), 0, s, d, mf, out, agent, k0);
+  }
+}
+
 // The IB of one step up to the marker forces.  hist_prev: see k_win_u3d.
 // pipe_step >= 0 (pipelined form): the window velocity of a step after the first
 // comes from the hand-off buffer, the force window is written with st_agent, this
@@ -488,16 +498,15 @@ void win_u_any(const StepCtx &c, const IB3DDev &d, const void *src, bool first, 
 int ib3d_phase(const StepCtx &c, const IB3DDev &d, const void *src, bool first, double *hist_prev, hipStream_t s,
                const float *halo = nullptr, int pipe_step = -1, double *hist = nullptr) {
   const unsigned gm = (unsigned)((d.M + 3) / 4), gc = (unsigned)((d.cells + 255) / 256);   // k_mark3d: 4 markers / block
-  const unsigned gs = (unsigned)((8 * d.cells + 255) / 256);                               // k_spread3d: 8 lanes / cell
   if (pipe_step > 0 && !first) hipLaunchKernelGGL(k_win_u3d_halo, dim3(gc), dim3(256), 0, s, d, halo, pipe_step);
   else win_u_any(c, d, src, first, hist_prev, s);
   hipLaunchKernelGGL(k_mark3d, dim3(gm), dim3(256), 0, s, d, 0);
   for (int it = 1; it < d.n_iter; ++it) {
-    hipLaunchKernelGGL(k_spread3d, dim3(gs), dim3(256), 0, s, d, (const float *)d.dF, d.acc, false);
+    launch_spread(d, d.dF, d.acc, false, s);
     hipLaunchKernelGGL(k_mark3d, dim3(gm), dim3(256), 0, s, d, it);
   }
   if (pipe_step >= 0) {
-    hipLaunchKernelGGL(k_spread3d, dim3(gs), dim3(256), 0, s, d, (const float *)d.F, d.g_win, true);
+    launch_spread(d, d.F, d.g_win, true, s);
     if (hist) hipLaunchKernelGGL(k_hist3d, dim3(1), dim3(256), 0, s, d, hist);
     hipLaunchKernelGGL(k_publish3d, dim3(1), dim3(1), 0, s, d, pipe_step);
   }
