@@ -153,7 +153,8 @@ typedef struct VsxIB3D {
   float ds;
   int32_t pipelined;          /* 1: the IB of step t + 1 runs on a second stream while the bulk
                                  pass of step t streams (needs `halo`, the window 2+ cells inside
-                                 the grid, and walls without shared corners)                   */
+                                 the grid, and walls without shared corners; a window whose
+                                 waiting blocks would fill the device runs as 0)               */
   float *g_win;               /* device [3][cells]: force window of the last step              */
   float *work;                /* device scratch, vsx_ib3d_work_floats(M, cells) floats           */
   double *hist_h;             /* optional device [n_steps][3]: total marker force (FP64)        */

@@ -310,14 +310,17 @@ def test_cells_on_several_walls(sim, shape, walls):
     assert_close(got, ref, 2e-5, f"{walls} {shape}")
 
 
-def test_sphere_window_of_several_spread_launches(sim):
-    """A window of more cells (130^3) than one launch of the spread takes (2^21).
-    Tolerances as in test_sphere_matches_oracle."""
+@pytest.mark.parametrize("pipelined", [False, True], ids=["sequential", "pipelined"])
+def test_sphere_window_of_several_spread_launches(sim, pipelined):
+    """A window of more cells (130^3) than one launch of the spread takes (2^21), and
+    of more waiting blocks than the device holds at once: the pipelined form runs it
+    sequentially.  Tolerances as in test_sphere_matches_oracle."""
     kw = dict(nx=140, ny=134, nz=134, D=124.0, cx=67.0, cy=67.0, cz=67.0, n_markers=48000)
     oc, pc = small_sphere(S.Sphere3D, **kw), small_sphere(sim.SphereCase, **kw)
     assert pc.ib_size ** 3 > 1 << 21
-    say(f"sphere window {pc.ib_size}^3")
-    solver = sim.Sphere3D(pc)
+    say(f"sphere window {pc.ib_size}^3 pipelined={pipelined}")
+    assert min(pc.ib_origin) >= 2
+    solver = sim.Sphere3D(pc, pipelined=pipelined)
     f0 = oc.initial_f(np.float64)
     got, hh = solver.run(dev(f0), 2)
     W, I = oc.stencil(np.float32)

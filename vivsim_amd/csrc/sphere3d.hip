@@ -554,6 +554,30 @@ int64_t halo_blocks(const StepCtx &c, const IB3DDev &d) {
   return (int64_t)(d.S[0] + 2) * (d.S[1] + 2) * (zb1 - zb0 + 1);
 }
 
+// Whether the kernels of the pipelined form that wait for one another leave room
+// for the kernels they wait for: the bulk blocks in the window hold their waves until
+// the IB kernels of their step are done, the first IB kernel of the next step its until that
+// bulk pass has handed over.  At most 8 waves of either kind per compute unit (2 per
+// SIMD, where the kernels' registers allow 4 and more).  Beyond that the waiting blocks of
+// a window of 130^3 held every slot of the chip until their bounded waits ran out.
+int pipe3d_fits(const StepCtx &c, const IB3DDev &d, bool *fits) {
+  static int units[64] = {0};
+  int dev = 0;
+  VSX_HIP(hipGetDevice(&dev));
+  VSX_REQUIRE(dev >= 0 && dev < 64, "device index %d out of range", dev);
+  if (units[dev] == 0) {
+    int v = 0;
+    VSX_HIP(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev));
+    units[dev] = v;
+  }
+  dim3 grid, block;
+  bulk_grid<D3Q19>(c, grid, block);
+  const int64_t zb = (d.org[2] + d.S[2] - 1) / (int)block.x - d.org[2] / (int)block.x + 1;
+  const int64_t bulk = (int64_t)d.S[0] * d.S[1] * zb * (block.x / 64), halo = (d.cells + 255) / 256 * 4;
+  *fits = bulk <= 8 * (int64_t)units[dev] && halo <= 8 * (int64_t)units[dev];
+  return VSX_OK;
+}
+
 int validate_ib3d(const VsxLbm *p, const VsxIB3D *ib) {
   if (!ib) return fail(VSX_ERR_VALUE, "null IB parameters");
   VSX_REQUIRE(ib->n_markers > 0, "marker count %d out of range", ib->n_markers);
@@ -594,6 +618,10 @@ int sphere_run(const VsxLbm *p, const VsxIB3D *ib, const float *f_in, float *f_o
     VSX_REQUIRE(!(p->n_walls > 0 && walls_need_edge<D3Q19>(*p)), "the pipelined sphere step needs walls without "
                 "shared corners");
     VSX_REQUIRE(ib->halo, "the pipelined sphere step needs the hand-off buffer ib->halo");
+  }
+  bool pipelined = ib->pipelined;
+  if (pipelined && (rc = pipe3d_fits(c, d, &pipelined))) return rc;
+  if (pipelined) {
     PipeRes *r = nullptr;
     if ((rc = pipe_res(&r))) return rc;
     const int n_halo = (int)halo_blocks(c, d);

@@ -445,7 +445,8 @@ class SphereCase:
 class Sphere3D:
     """Device state and fused run of a ``SphereCase`` (``vsx_sphere3d_run``).
     pipelined=True (the window 2+ cells inside the grid): the IB of step t + 1
-    runs on a second stream while the bulk pass of step t streams.  The
+    runs on a second stream while the bulk pass of step t streams (windows whose
+    waiting blocks would fill the device run sequentially).  The
     default is the sequential form: the sphere's IB kernels are multi-
     workgroup kernels that, run beside the bulk pass, get too few compute
     units and make the pipelined step slower (0.24 against 0.15 ms at
