@@ -10,7 +10,7 @@ from tests.gpu_util import say
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx,ny,storage,tol", [(2048, 2048, "f32", 1e-5), (2048, 1990, "f32", 1e-5),
+@pytest.mark.parametrize("nx,ny,storage,tol", [(2048, 2048, "f32", 1e-5), (2048, 1990, "f32", 1e-5), (1500, 1500, "f16s", 1e-3),
                                                (4096, 4096, "f16s", 1e-3)])
 @pytest.mark.parametrize("d0", [0.96, 0.9, 0.8])
 def test_moving_window_crosses_a_tile_edge(gpu_lib, nx, ny, storage, tol, d0):

@@ -169,11 +169,12 @@ struct Streamed : B {
 // last-level cache holds.  A launch ends with the write-back of what its XCDs'
 // L2s (8 x 4 MB) hold dirty, and the next launch waits for it; written through,
 // the cells leave while the launch still runs.  Rows of whole 128-byte lines
-// only: a partial line written through costs a transfer of its own.  us per
-// step, plain against written through: VIV 1024^2 FP32 22.4 -> 20.5, 2048^2 FP32
-// 66.7 -> 62.3, 1024^2 FP16S 19.8 -> 18.8; plain step 64^3 9.9 -> 8.1; with rows
-// of 1500 cells 33.2 -> 33.7, of 127 cells 77.8 -> 81.8; above the last-level cache
-// (3000^2) 143 -> 163.
+// only: a partial line written through costs a transfer of its own (small VIV fields
+// have a rule of their own, kThroughAnyRowBytes).  us per step, plain against written
+// through: VIV 1024^2 FP32 21.4 -> 19.8, 2048^2 FP32 62.8 -> 59.4, 1024^2 FP16S
+// 19.7 -> 18.6; periodic 96^3 25.0 -> 24.2, 128^3 69.8 -> 68.5; with rows of 1500 cells
+// (VIV 1500^2) 31.1 -> 32.3, of 1501 (1999 x 1501) 40.1 -> 43.0, of 127 (3D) 77.8 -> 81.8; above
+// the last-level cache (3000^2) 143 -> 163.
 template <class B>
 struct Through : B {
   using T = typename B::T;

@@ -405,6 +405,16 @@ Tiles make_tiles(const StepCtx &c);
 // shorter; FP32 tiles stay single (no gain at 4096^2, a loss at 1024^2).
 constexpr int kPairMinTiles = 4096;
 
+// Fields up to this size are written through whatever their rows.  There the IB chain
+// bounds the step, and what the bulk pass leaves to do between two passes counts: with
+// plain stores the next pass's opening burst falls on the IB kernel's pull of the
+// window (1.6 us of the chain, 2.7 in the burst), while the dearer stores are hidden.
+// us per step, plain against written through, unaligned rows: FP32 640 x 500 19.9, 18.6;
+// 900 x 1000 21.0, 19.9; 1024 x 1000 21.1, 20.0; 1024 x 1023 21.9, 20.4; 1300 x 1100 (51 MB)
+// 22.6, 22.7; 1500^2 31.1, 32.3; FP16S 1000^2 19.8, 18.5; 1500 x 1300 (35 MB) 26.7, 26.5;
+// 1500^2 (40 MB) 27.3, 27.8.
+constexpr size_t kThroughAnyRowBytes = size_t(36) << 20;
+
 template <class SRC, class DST, int COLL, bool PAIR, int MODE>
 int launch_fused_p(const StepCtx &c, const VsxIB2D &ib, const void *src, void *dst, int step, hipStream_t s,
                    const Tiles &T) {
@@ -439,12 +449,14 @@ int launch_fused_c(const StepCtx &c, const VsxIB2D &ib, const void *src, void *d
     // full steps of the pipelined form: non-temporal field stores when the work
     // buffer alone exceeds the last-level cache (such a 16-bit field has more
     // than kPairMinTiles tiles, so its bulk blocks take tile pairs), written
-    // through below it
+    // through below it where the rows or the size allow
     if (ib.fused == 2 && (size_t)c.n * 9 * sizeof(typename DST::T) > kLastLevelCacheBytes)
       return launch_fused_p<SRC, Streamed<DST>, COLL, sizeof(typename SRC::T) == 2, MODE>(c, ib, src, dst, step, s, T);
   }
   if constexpr (MODE == kModeFull) {
-    if (ib.fused == 2 && write_through(c.n, 9, c.dims[1], sizeof(typename DST::T)) &&
+    const bool through = write_through(c.n, 9, c.dims[1], sizeof(typename DST::T)) ||
+                         (size_t)c.n * 9 * sizeof(typename DST::T) <= kThroughAnyRowBytes;
+    if (ib.fused == 2 && through &&
         !(sizeof(typename SRC::T) == 2 && T.ntx * T.nty >= kPairMinTiles))
       return launch_fused_p<SRC, Through<DST>, COLL, false, MODE>(c, ib, src, dst, step, s, T);
   }
