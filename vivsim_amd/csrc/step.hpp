@@ -22,6 +22,7 @@
 // (on walls of several axes) go to the first blocks of the same launch, a group
 // of 2^D lanes per cell (edge_cells); they exist only when such cells do.
 #pragma once
+#include <cstddef>
 #include <type_traits>
 #include <utility>
 
@@ -69,27 +70,30 @@ __device__ __forceinline__ void gather_cell3(const float *__restrict__ mf, const
   }
 }
 
-// Whole lines of the argument segment: every wave waits for the lines that hold
-// the grid's size and the pointers behind it before its first load.
+// Every wave waits for the lines of the argument segment that it reads before its
+// first load, so what all kernels read there shares one line: the grid, the walls'
+// order and the window's pointers.  The whole fills lines too.
 struct alignas(64) StepCtx {
   VsxLbm p;
-  Window win;
-  int32_t dims[3];         // nx, ny, nz (nz = 1 in 2D)
-  int64_t n;               // cells
+  alignas(64) int32_t dims[3];   // nx, ny, nz (nz = 1 in 2D)
   // Walls by location, so device code indexes walls only by compile-time
   // location: order[LOC] = position of the wall at LOC in p.walls (-1: none,
   // -2: several walls at LOC), at[LOC] = that wall.
   int32_t order[6];
+  int64_t n;               // cells
+  Window win;
   VsxWall at[6];
   float shift[19];         // 16-bit storage: stored value = f_i - shift[i] = f_i - feq_i(1, p.store_u)
 };
+static_assert(offsetof(StepCtx, win) % 64 + 2 * sizeof(void *) <= 64, "win.origin and win.g on the line of dims");
 
 // 3D steps: the forces `F` [M][3] of the markers, gathered by the window's cells
 // themselves (null: read from win.g); stencil weights and cell -> slot lists of
 // vsx_ib3d_transpose_stencil; also stored in win.g.  Behind the rest, and in 3D only:
-// within Window these 32 bytes moved the grid's size across a line (periodic 3D runs, us
-// per step, within Window -> here: 32^3 4.47 -> 3.92, 64^3 9.01 -> 8.81, 65 x 64 x 63
-// 11.55 -> 11.37, 96^3 24.4 -> 24.2).
+// within Window these 32 bytes moved fields across lines (us per step, within Window ->
+// here and dims .. win.g on one line: periodic 32^3 KBC 4.64 -> 4.44, 64^3 9.00 -> 8.85,
+// 65 x 64 x 63 11.56 -> 11.37, 96^3 24.5 -> 24.2, batch of 64 244.0 -> 239.8; with dims and order on
+// two lines a 96 x 65 channel x 20 took 68.9 us instead of 67.9).
 struct StepCtx3 : StepCtx {
   const float *F = nullptr, *W = nullptr;
   const int32_t *cell_ptr = nullptr, *cell_slot = nullptr;
