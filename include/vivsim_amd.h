@@ -115,8 +115,8 @@ typedef struct VsxIB2D {
                           workgroup of step t has pulled its window (fused == 1: the bulk
                           tiles wait for it) or once the bulk pass of step t has handed the
                           cells around the window to the next IB kernel (fused == 2);
-                          [7] = step0 + t + 1 once the bulk pass of step t (0 or 1) of a run
-                          has begun (fused == 2)                                             */
+                          [7] = step0 + 1 once the first bulk pass of a run has begun
+                          (fused == 2)                                                       */
   int32_t step0;       /* global index of the first step of this run (0 after a reset of the
                           body state, which must also zero win_origin)                       */
   int32_t fused;       /* 0: separate IB and bulk kernels; 1: one launch per step, the IB
@@ -128,7 +128,7 @@ typedef struct VsxIB2D {
   float *halo;         /* device [2][9][win + 4][win + 4] FP32 (fused == 2): post-collision
                           populations around the window, handed from the bulk pass of a step
                           to the IB kernel of the next (half (step0 + t) & 1 by step t); the
-                          first six words hold window origins                               */
+                          first four words hold window origins                              */
   int32_t *status;     /* optional pinned host int32 (hipHostMalloc) or NULL: the kernels also
                           store their error codes there (1 = a bounded wait ran out, 2 = the
                           pipelined window left the hand-off buffer), so a host can check a

@@ -69,6 +69,16 @@ int fused_full(const StepCtx &c, const VsxIB2D &ib, const void *src, void *dst, 
   return fused_mode_any<kModeFull>(c, ib, src, dst, step, s);
 }
 
+// Window origin of a run's first pass into its slot, from the body state that the
+// caller's stream holds (the caller may have set it since the last run).
+__global__ void k_first_origin(StepCtx c_arg, VsxIB2D ib) {
+  if (threadIdx.x != 0) return;
+  int o[4];
+  window_origin(kernel_ctx(), ib, ib.body + 6 * (ib.step0 & 1), o);
+  int32_t *r = origin_slot(ib, ib.step0);
+  r[0] = o[2];
+  r[1] = o[3];
+}
 
 int viv_run(const VsxLbm *p, const VsxIB2D *ib_in, const float *f_in, float *f_out, void *wa, void *wb, int n,
             void *stream) {
@@ -112,6 +122,11 @@ int viv_run(const VsxLbm *p, const VsxIB2D *ib_in, const float *f_in, float *f_o
     VSX_REQUIRE(ib->halo, "the pipelined VIV step needs the hand-off buffer ib->halo");
     PipeRes *r = nullptr;
     if ((rc = pipe_res(&r))) return rc;
+    ib_dev.reserved = n == 1;   // the kernels' view: no k_first_origin (3.3 us of a one-step run's 40)
+    if (n > 1) {
+      hipLaunchKernelGGL(k_first_origin, dim3(1), dim3(64), 0, s, c, *ib);
+      VSX_CHECK_LAUNCH();
+    }
     for (int t = 0; t < n; ++t) {
       if ((rc = launch_ib_pipe(c, *ib, f_in, t == 0, t, r->s))) return rc;
       void *dst = (push && t == n - 1) ? f_out : bufs[t & 1];

@@ -53,15 +53,14 @@ __device__ __forceinline__ void window_origin(const StepCtx &c, const VsxIB2D &i
 }
 
 // Pipelined form: clamped window origin of step gstep, for the bulk pass of that
-// step (but for a run's first, which reads the body state).  Three slots by gstep: the
-// IB kernel of step g writes the next step's, after the hand-off of pass g - 1, so
-// while pass g may run beside it, and pass g - 2, whose slot that is, has ended.  (The two
-// body slots do not do: the IB kernel of step g + 1 ends while pass g still runs and
-// writes the one that pass g started from.)  The slots are the first words of
-// the hand-off buffer: populations at rest of the first row of its box, which no
-// window pulls (the window lies one cell and more inside) and the passes leave out.
+// step.  Two slots by gstep: the last hand-off tile of a pass writes the next pass's
+// (count_halo_tile), k_first_origin that of a run's first.  (The body state does not
+// do: the IB kernel of step g + 1 ends while pass g still runs and writes the slot
+// that holds the state before step g.)  The slots are the first words of the hand-off
+// buffer: populations at rest of the first row of its box, which no window pulls (the
+// window lies one cell and more inside) and the passes leave out.
 __device__ __forceinline__ int32_t *origin_slot(const VsxIB2D &ib, int gstep) {
-  return reinterpret_cast<int32_t *>(ib.halo) + 2 * (gstep % 3);
+  return reinterpret_cast<int32_t *>(ib.halo) + 2 * (gstep & 1);
 }
 
 // Window velocity of a cell that lies on a domain wall (rare: only when the IB
@@ -1245,13 +1244,11 @@ constexpr int kWinHalo = 2;    // pull from the FP32 hand-off buffer `halo` [9][
 // ONE: the two components of the multi-direct forcing one after the other on one
 // plane of the grid (they share the weights only): 10 S^2 instead of 16 S^2 bytes
 // of LDS for a longer loop.
-// RING: also writes the next step's window origin to its slot (origin_slot).
-template <class SRC, int WSRC, int UW, int TAG, bool SPLIT = false, int TPM = 0, bool ONE = false, bool RING = false>
+template <class SRC, int WSRC, int UW, int TAG, bool SPLIT = false, int TPM = 0, bool ONE = false>
 __device__ __forceinline__ void ib_atomic(const StepCtx &c, const VsxIB2D &ib, const typename SRC::T *__restrict__ src,
                                           const float *halo, int hidx, int gstep, int32_t *go_flag,
                                           const double *body_in, double *body_out, float *lds,
-                                          int32_t *wait_flag = nullptr, int wait_target = 0,
-                                          int32_t *free_flag = nullptr, int free_target = 0) {
+                                          int32_t *wait_flag = nullptr, int wait_target = 0) {
   const int S = ib.win, SS = S * S, M = ib.n_markers;
   __shared__ double s_body[6];
   __shared__ int s_org[6];
@@ -1495,15 +1492,6 @@ __device__ __forceinline__ void ib_atomic(const StepCtx &c, const VsxIB2D &ib, c
     s_red[0][tid >> 6] = hx;
     s_red[1][tid >> 6] = hy;
   }
-  // the largest origins, read here: behind the Newmark step that load is waited for
-  int hi0 = 0, hi1 = 0;
-  if constexpr (RING) {
-    hi0 = c.dims[0] - S;
-    hi1 = c.dims[1] - S;
-    asm volatile("" : "+s"(hi0), "+s"(hi1));
-  }
-  // body_out may have readers left: the last wave waits for them while the others sum
-  if (free_flag && tid == nt - 64) spin_until(ib, free_flag, free_target);
   __syncthreads();
   if (tid == 0) {
     double h[2] = {0.0, 0.0};
@@ -1525,12 +1513,6 @@ __device__ __forceinline__ void ib_atomic(const StepCtx &c, const VsxIB2D &ib, c
       out[4 + k] = on ? c2 * an + v2 : 0.0;
     }
     for (int k = 0; k < 6; ++k) __hip_atomic_store(&body_out[k], out[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if constexpr (RING) {
-      int32_t *r = origin_slot(ib, gstep + 1);   // as window_origin
-      const int x = min(max((int)trunc(ib.win_x0 + out[4]), 0), hi0), y = min(max((int)trunc(ib.win_y0 + out[5]), 0), hi1);
-      __hip_atomic_store(&r[0], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&r[1], y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
     if (ib.hist_d && hidx >= 0) {
       __hip_atomic_store(&ib.hist_d[2 * hidx], out[4], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(&ib.hist_d[2 * hidx + 1], out[5], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1590,8 +1572,10 @@ __device__ __forceinline__ void count_window_tile(const VsxIB2D &ib, int gstep, 
 // Pipelined form: once every thread's hand-off stores have completed, count
 // the tile in ib.win_origin[4]; the last of the n hand-off tiles of step gstep
 // resets the counter (the next step's tiles run in a later launch of the same
-// stream) and raises ib.win_origin[6] to gstep + 1.
-__device__ __forceinline__ void count_halo_tile(const VsxIB2D &ib, int gstep, int n) {
+// stream), raises ib.win_origin[6] to gstep + 1 and leaves the next pass its window
+// origin: the force-window tiles among the n have waited for this step's IB kernel,
+// which had written the next body state by then.
+__device__ __forceinline__ void count_halo_tile(const StepCtx &c, const VsxIB2D &ib, int gstep, int n) {
   wait_mem();
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -1599,6 +1583,14 @@ __device__ __forceinline__ void count_halo_tile(const VsxIB2D &ib, int gstep, in
     if (before == n - 1) {
       __hip_atomic_store(&ib.win_origin[4], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(&ib.win_origin[6], gstep + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      double *next = ib.body + 6 * ((gstep + 1) & 1), b[6];
+      b[4] = __hip_atomic_load(next + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      b[5] = __hip_atomic_load(next + 5, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      int o[4];
+      window_origin(c, ib, b, o);
+      int32_t *r = origin_slot(ib, gstep + 1);
+      r[0] = o[2];
+      r[1] = o[3];
     }
   }
 }

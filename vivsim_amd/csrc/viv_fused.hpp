@@ -140,6 +140,12 @@ k_viv_fused(StepCtx c_arg, VsxIB2D ib, const typename SRC::T *__restrict__ src, 
   const int gstep = ib.step0 + step, slot = gstep & 1;
   const double *body_in = ib.body + 6 * slot;
   constexpr bool pipe = PIPE;
+  if constexpr (MODE == kModeFirst) {
+    // pipelined run: the caller's earlier work on this stream is complete; let
+    // the run's first IB kernel start
+    if (pipe && blockIdx.x == 0 && threadIdx.x == 0)
+      __hip_atomic_store(&ib.win_origin[7], gstep + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   if constexpr (!pipe) {
     if (blockIdx.x == 0) {
       ib_atomic<SRC, MODE == kModeFirst ? kWinLocal : kWinPull, 2, 1>(c, ib, src, nullptr, step, gstep,
@@ -151,16 +157,16 @@ k_viv_fused(StepCtx c_arg, VsxIB2D ib, const typename SRC::T *__restrict__ src, 
   }
   // The window origin.  All blocks need the same one: a block with another takes its
   // tile from another order, and some tiles are then taken by no block.  One-launch
-  // form and first pass of a run: from the body state, which the previous launch wrote
-  // (this one writes the other slot; pipelined, the IB kernel of the run's second
-  // step is the next to write this one, once the run's second pass has begun: win_origin[7]).
-  // Later passes: from origin_slot, written by the IB kernel of the previous step,
-  // which the previous launch waited for.  Either is complete before the launch
-  // starts, so every wave reads it through the scalar cache: read at agent scope by
-  // one thread and passed through LDS and a barrier, it kept every tile from issuing
-  // its loads for a memory round trip (4096 x 4096 FP16S: 151 -> 145 us per step).
+  // form: from the body state, which the previous launch wrote (this one writes the
+  // other slot).  Pipelined form: from origin_slot, which the previous launch wrote, or, in
+  // a run of one step (ib.reserved), from the body state, as no IB kernel writes its slot
+  // before the next run's first pass.
+  // Either is complete before the launch starts, so every wave reads it through the
+  // scalar cache: read at agent scope by one thread and passed through LDS and a
+  // barrier, it kept every tile from issuing its loads for a memory round trip
+  // (4096 x 4096 FP16S: 151 -> 145 us per step).
   int o4[4];
-  if constexpr (pipe && MODE != kModeFirst) {
+  if (pipe && !(MODE == kModeFirst && ib.reserved)) {
     const int32_t *r = origin_slot(ib, gstep);
     o4[2] = r[0];
     o4[3] = r[1];
@@ -220,10 +226,6 @@ k_viv_fused(StepCtx c_arg, VsxIB2D ib, const typename SRC::T *__restrict__ src, 
     // tile around the window (pipelined form): collide (after the force window
     // when the tile intersects it), store, hand the cells within 2 of the window
     // to the next step's IB kernel
-    // block 0 of a run's first and second pass: everything earlier on this stream is
-    // complete (kept out of the other blocks' way: 4096 x 4096 FP16S 147 -> 143 us per step)
-    if (step <= 1 && blockIdx.x == 0 && threadIdx.x == 0)
-      __hip_atomic_store(&ib.win_origin[7], gstep + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int S = ib.win;
     const bool force = tx * T.TX < org[0] + S && (tx + 1) * T.TX > org[0] && ty * T.TY < org[1] + S &&
                        (ty + 1) * T.TY > org[1];
@@ -243,7 +245,7 @@ k_viv_fused(StepCtx c_arg, VsxIB2D ib, const typename SRC::T *__restrict__ src, 
         for (int q = 0; q < 9; ++q)
           if (q > 0 || a > 0) st_agent(&h[q * EE + a * E + b], DST::rt(f[q], c.shift[q]));   // (origin_slot)
       }
-      count_halo_tile(ib, gstep, n_win);
+      count_halo_tile(c, ib, gstep, n_win);
     }
     return;
   }
@@ -296,12 +298,11 @@ __global__ __launch_bounds__(kIbThreads) void k_ib_pipe(StepCtx c_arg, VsxIB2D i
   // zeroed grid) is done while the previous step's bulk pass still streams;
   // the pull waits for that pass's hand-off flag
   // (the first IB kernel of a run waits for the run's first bulk pass to start:
-  // ib.win_origin[7] = step0 + 1; the second writes the body slot that this pass
-  // reads until its end, and waits for the second pass to start)
-  ib_atomic<Store<VSX_STORE_F32>, WSRC, 2, 2, true, TPM, false, true>(
-      c, ib, src, halo, step, gstep, nullptr, ib.body + 6 * slot, ib.body + 6 * (slot ^ 1), lds,
-      WSRC == kWinHalo ? &ib.win_origin[6] : &ib.win_origin[7], WSRC == kWinHalo ? gstep : gstep + 1,
-      step == 1 ? &ib.win_origin[7] : nullptr, gstep + 1);
+  // ib.win_origin[7] = step0 + 1)
+  ib_atomic<Store<VSX_STORE_F32>, WSRC, 2, 2, true, TPM>(c, ib, src, halo, step, gstep, nullptr, ib.body + 6 * slot,
+                                                     ib.body + 6 * (slot ^ 1), lds,
+                                                     WSRC == kWinHalo ? &ib.win_origin[6] : &ib.win_origin[7],
+                                                     WSRC == kWinHalo ? gstep : gstep + 1);
   publish_ready(ib, gstep + 1);
 }
 
