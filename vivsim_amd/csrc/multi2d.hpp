@@ -50,7 +50,9 @@ struct MultiCfg {
   static_assert(NT % 64 == 0 && NT / 64 >= (RX > 64 || RW > 64 ? 12 : 8), "a wave for every wall and corner unit");
 };
 
-// The region in LDS is updated in place.  After an odd operation s population i
+// The region in LDS is updated in place (the AA pattern: Bailey, Myre, Walsh, Lilja, Saar,
+// "Accelerating lattice Boltzmann fluid flow simulations using graphics processors",
+// ICPP 2009).  After an odd operation s population i
 // of cell x lies at b[i][x]; the next one pulls b[i][x - c_i] and writes its
 // result to b[opp i][x + c_i], the places it read; the one after that finds
 // its pulled populations at b[opp i][x] and writes b[i][x].  So the cells of an
@@ -298,6 +300,8 @@ int run_multi(const StepCtx &c, const float *f_in, float *f_out, void *wa, void 
 // 8.2; 362^2 4.9 | 4.3 | 5.9 and 9.1; 512^2 6.9 | 5.5 | 5.9 and 11.2; 1031 x 777
 // 18.0 | 12.3 | 8.0 and 15.0; 4000 x 2050 158 | 100 | 51 and 145; FP16S 1031 x 777
 // 8.7 | 9.7 (20 x 64 | 40 x 64) and 11.2; 2048^2 29.3 | 26.4 and 32.9; 4000 x 2050 54.8 | 48.3 and 78.
+// What bounds the large tiles is VALU issue: at 4000 x 2050 FP32 BGK it is busy throughout, LDS 23 %
+// of the time, HBM at 31 % of peak; 237 instructions per cell and operation, rings included.
 // Six operations per launch: with four the large tiles took 60 us at 4000 x 2050.
 template <int COLL, class ST>
 int run_multi_tiles(const StepCtx &c, const float *f_in, float *f_out, void *wa, void *wb, int n, hipStream_t s) {

@@ -185,7 +185,8 @@ int multi2d_run_e3m12(const StepCtx &, const float *, float *, void *, void *, i
 
 // Whether a run goes through them: sides that hold the seam and its rings inside
 // a tile, at most one wall per face, and no launch (run_multi) that reads a buffer
-// it writes.  Single passes also take an input that is work_a (collided in place) and
+// it writes.  (Sides from 22 on would hold the seam and its rings without meeting
+// their own copy; below 40 that has been neither tested nor timed.)  Single passes also take an input that is work_a (collided in place) and
 // an output that is the work buffer idle at the end.
 inline bool multi2d_takes(const StepCtx &c, const float *f_in, const float *f_out, const void *wa, const void *wb,
                           int n) {
