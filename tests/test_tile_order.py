@@ -1,8 +1,8 @@
 """CPU check of the tile order of the fused VIV passes (``window_tiles`` and
 ``tile_of_block`` of csrc/viv2d.hpp, compiled for the host): with one window
 origin, the blocks of a launch take every tile once.  With the origin of a
-later step in some of the blocks they do not, so the body state that a pass
-derives its origin from must not change while the pass runs."""
+later step in some of the blocks they do not, so what a pass takes its origin
+from must not change while the pass runs."""
 
 import os
 import subprocess
